@@ -1027,13 +1027,16 @@ void choose_variant(agpt_attn_s* h, int& tile) {
                     (hg * hd * elem) % 16 == 0 && h->fwd_lds <= static_cast<size_t>(bbudget) &&
                     h->bq_lds <= static_cast<size_t>(bbudget) && h->kv_lds <= static_cast<size_t>(bbudget);
     if (h->fused && h->fb_lds > static_cast<size_t>(bbudget)) h->fused = false;
-    // Path carry (head_dim 16: its dQ registers fit) when its LDS keeps the
-    // workgroups per CU (registers hold the one-pass backward to two).
+    // Path carry when its LDS keeps the workgroups per CU (registers hold the
+    // one-pass backward to two). At head_dim 32 (one head per workgroup) it
+    // also brings the second workgroup: the dQ sums sit in registers instead
+    // of 32 KB of LDS tiles, and no prefix partials go through HBM (767K
+    // rows, 4 x 32, depth 32, seeds and RoPE: backward 2.40 -> 1.90 ms).
     {
       const size_t tabs = sizeof(agpt_blk::BlockTables<2>);
       auto per_cu = [&](size_t b) { return static_cast<size_t>(lim) / ((b + tabs + 511) & ~static_cast<size_t>(511)); };
       const size_t with = agpt_blk::fused_lds_bytes(h->max_depth, h->fhg, hd, true);
-      h->carry = h->fused && hd == 16 && env_int("AGPT_ATTN_CARRY", 1) != 0 &&
+      h->carry = h->fused && env_int("AGPT_ATTN_CARRY", 1) != 0 &&
                  per_cu(with) >= std::min<size_t>(per_cu(h->fb_lds), 2) && per_cu(with) >= 1;
       if (h->carry) h->fb_lds = with;
     }
@@ -1804,20 +1807,15 @@ void launch_bwd(const agpt_attn_s* h, const void* q, const void* k, const void* 
         }
       };
       with_124(h->fhg, [&](auto hgc) {
-        if constexpr (HD == 16) {
-          if (h->carry) {
-            run(hgc, std::true_type{});
-            return;
-          }
-        }
-        run(hgc, std::false_type{});
+        if (h->carry) run(hgc, std::true_type{});
+        else run(hgc, std::false_type{});
       });
       pm.mark(1);
       fused_done = true;
       if (h->carry) {
         pm.mark(2);
         pm.mark(3);
-        if (HD == 16 && h->n_chunks_sched > 1)
+        if (h->n_chunks_sched > 1)
           hipLaunchKernelGGL((agpt_blk::bwd_carry_kernel<HD, PlanDev, RopeArgs>), dim3(h->n_chunks_sched - 1),
                              dim3(256), 0, st, plan_dev(h), h->d_E, h->d_F, dk, dv, acc_dk, acc_dv, rope,
                              h->cfg.n_heads);

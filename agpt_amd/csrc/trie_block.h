@@ -1135,8 +1135,14 @@ __host__ __device__ inline size_t fused_lds_bytes(int max_depth, int HG, int HD,
          (carry ? carry_bytes(max_depth, HG, HD) : static_cast<size_t>(kWaves) * kTile * HD * sizeof(float));
 }
 
+// Waves per SIMD the register allocator must leave room for: two where the
+// LDS holds two workgroups at depth 32 and the kernel would else go past 256
+// VGPRs by a few (head_dim 32 with the carry).
+template <int HD, int HG, bool kCarry>
+constexpr int kBwdWaves = HD == 32 && HG == 1 && kCarry ? 2 : 1;
+
 template <int HD, typename Tin, int HG, bool kCarry, typename PlanT, typename RopeT>
-__global__ __launch_bounds__(kThreads) void bwd_kernel(
+__global__ __launch_bounds__(kThreads, (kBwdWaves<HD, HG, kCarry>)) void bwd_kernel(
     PlanT pl, const Tin* __restrict__ Q, const Tin* __restrict__ K, const Tin* __restrict__ V,
     const Tin* __restrict__ O, const float* __restrict__ lse, const Tin* __restrict__ dO,
     float* __restrict__ dQ, float* __restrict__ dK, float* __restrict__ dV, float* __restrict__ Pk,
@@ -1267,20 +1273,29 @@ __global__ __launch_bounds__(kThreads) void bwd_kernel(
         load_vec<KD>(Gs + qr * WS + hoff + KD * g, ga);
         const f4 l2v = *reinterpret_cast<const f4*>(&tb.l2[hh][q0]);
         const f4 dlv = *reinterpret_cast<const f4*>(&tb.dl[hh][q0]);
+        auto columns = [&] {
 #pragma unroll
-        for (int j = 0; j < MT; ++j)
+          for (int j = 0; j < MT; ++j)
 #pragma unroll
-          for (int r = 0; r < 4; ++r) {
-            const int row = (q0 + r) * WS + hoff + kBlk * j + c;
-            gcol[j][r] = ld1(Gs + row);
-            qcol[j][r] = ld1(Qs + row);
-          }
+            for (int r = 0; r < 4; ++r) {
+              const int row = (q0 + r) * WS + hoff + kBlk * j + c;
+              gcol[j][r] = ld1(Gs + row);
+              qcol[j][r] = ld1(Qs + row);
+            }
+        };
+        if constexpr (MT == 1) columns();
         __builtin_amdgcn_sched_barrier(0);  // (the scheduler would sink them past the S products)
         f4 sv = f4{0.0f, 0.0f, 0.0f, 0.0f}, tv = sv;
 #pragma unroll
         for (int j = 0; j < KD; ++j) {
           sv = mfma16(qa[j], kf[j], sv);  // sv[r]: query q0+r against key kslot
           tv = mfma16(ga[j], vf[j], tv);
+        }
+        // At hd 32 the columns take the registers of the row slices, which
+        // the products above have read (all at once they spill).
+        if constexpr (MT > 1) {
+          __builtin_amdgcn_sched_barrier(0);
+          columns();
         }
         float p[4], ds[4];
 #pragma unroll
