@@ -225,6 +225,7 @@ struct RopeArgs {
   const float* cos_t;
   const float* sin_t;
   int seq_len;
+  int lds_rows;  // block backward: rotations of depths 1..lds_rows staged in LDS (0: none)
 };
 
 __device__ __forceinline__ int rope_pos(int depth, int seq_len) {
@@ -702,6 +703,7 @@ struct agpt_attn_s {
   bool fused = false;           // block kernels: one-pass backward (fp32)
   int fhg = 1;                  // heads per workgroup of the one-pass backward
   bool carry = false;           // one-pass backward carries path sums (E, F replace Pk, Pv)
+  bool rope_lds = false;        // block backward: the rotations fit in LDS at the same workgroups per CU
   bool deep = false;            // block kernels at head_dim 64: streamed key set (trie_deep.h)
   bool deep_carry = false;      // deep key side carries path sums (E, F replace Pk, Pv)
   bool dq_one_pass = true;      // deep bf16 dQ kernel: δ and dQ in one pass over the keys
@@ -1039,6 +1041,22 @@ void choose_variant(agpt_attn_s* h, int& tile) {
       h->carry = h->fused && env_int("AGPT_ATTN_CARRY", 1) != 0 &&
                  per_cu(with) >= std::min<size_t>(per_cu(h->fb_lds), 2) && per_cu(with) >= 1;
       if (h->carry) h->fb_lds = with;
+    }
+    // The inverse RoPE of the backward from a table in LDS: read from the
+    // caller's tables, each use would wait (the memory counter retires in
+    // order) for the next tile's prefetch issued before it. 3.2M rows, 8 x 16
+    // fp32, depth 32: backward 4.55 -> 3.93 ms (3.90 without RoPE). Where the
+    // table would cost a workgroup per CU it stays out.
+    {
+      const size_t rope = agpt_blk::rope_lds_bytes(h->max_depth, hd);
+      auto keeps = [&](size_t b, size_t tabs, size_t cap) {
+        auto n = [&](size_t x) { return std::min(cap, static_cast<size_t>(lim) / ((x + tabs + 511) & ~static_cast<size_t>(511))); };
+        return n(b + rope) >= n(b) && n(b + rope) >= 1;
+      };
+      h->rope_lds = env_int("AGPT_ATTN_ROPELDS", 1) != 0 &&
+                    (h->fused ? keeps(h->fb_lds, sizeof(agpt_blk::BlockTables<2>), 2)
+                              : keeps(h->bq_lds, sizeof(agpt_blk::BlockTables<4>), 4) &&
+                                    keeps(h->kv_lds, sizeof(agpt_blk::BlockTables<4>), 4));
     }
     if (ok) return;
     h->variant = 5;  // try the chain-group walk
@@ -1790,6 +1808,9 @@ void launch_bwd(const agpt_attn_s* h, const void* q, const void* k, const void* 
   const int D = h->cfg.n_heads * HD;
   pm.mark(0);
   bool fused_done = false;
+  // LDS of the block backward's rotation table (see choose_variant).
+  rope.lds_rows = rope.cos_t && h->rope_lds && h->variant == 6 && !h->deep ? h->max_depth : 0;
+  const size_t rope_extra = rope.lds_rows ? agpt_blk::rope_lds_bytes(h->max_depth, HD) : 0;
   if constexpr ((HD == 16 || HD == 32) && std::is_same<Tin, float>::value) {
     if (h->variant == 6 && h->fused) {
       clear_sched(h, st);
@@ -1798,8 +1819,9 @@ void launch_bwd(const agpt_attn_s* h, const void* q, const void* k, const void* 
         constexpr bool kCarry = decltype(cc)::value;
         if constexpr (HG <= 2) {
           auto fb = agpt_blk::bwd_kernel<HD, Tin, HG, kCarry, PlanDev, RopeArgs>;
-          set_lds(fb, h->fb_lds);
-          hipLaunchKernelGGL(fb, dim3(stream_grid(h, fb, h->fb_lds, HG)), dim3(agpt_blk::kThreads), h->fb_lds,
+          const size_t lds = h->fb_lds + rope_extra;
+          set_lds(fb, lds);
+          hipLaunchKernelGGL(fb, dim3(stream_grid(h, fb, lds, HG)), dim3(agpt_blk::kThreads), lds,
                              st, plan_dev(h), static_cast<const Tin*>(q), static_cast<const Tin*>(k),
                              static_cast<const Tin*>(v), static_cast<const Tin*>(o), lse,
                              static_cast<const Tin*>(dO), dq, dk, dv, kCarry ? h->d_E : h->d_Pk,
@@ -1942,15 +1964,16 @@ void launch_bwd(const agpt_attn_s* h, const void* q, const void* k, const void* 
         constexpr int HG = decltype(hgc)::value, UH = decltype(uhc)::value;
         if constexpr (block_shape_ok(HD, HG, UH)) {
           auto fq = agpt_blk::bwd_q_kernel<HD, Tin, HG, UH, PlanDev, RopeArgs>;
-          set_lds(fq, h->bq_lds);
-          hipLaunchKernelGGL(fq, dim3(stream_grid(h, fq, h->bq_lds)), dim3(agpt_blk::kThreads), h->bq_lds,
+          const size_t q_lds = h->bq_lds + rope_extra, kv_lds = h->kv_lds + rope_extra;
+          set_lds(fq, q_lds);
+          hipLaunchKernelGGL(fq, dim3(stream_grid(h, fq, q_lds)), dim3(agpt_blk::kThreads), q_lds,
                              st, plan_dev(h), static_cast<const Tin*>(q), static_cast<const Tin*>(k),
                              static_cast<const Tin*>(v), static_cast<const Tin*>(o), lse,
                              static_cast<const Tin*>(dO), dq, h->d_Dl, rope, h->cfg.n_heads, scale);
           pm.mark(1);
           auto fk = agpt_blk::bwd_kv_kernel<HD, Tin, HG, UH, PlanDev, RopeArgs>;
-          set_lds(fk, h->kv_lds);
-          hipLaunchKernelGGL(fk, dim3(stream_grid(h, fk, h->kv_lds)), dim3(agpt_blk::kThreads), h->kv_lds,
+          set_lds(fk, kv_lds);
+          hipLaunchKernelGGL(fk, dim3(stream_grid(h, fk, kv_lds)), dim3(agpt_blk::kThreads), kv_lds,
                              st, plan_dev(h), static_cast<const Tin*>(q), static_cast<const Tin*>(k),
                              static_cast<const Tin*>(v), lse, h->d_Dl, static_cast<const Tin*>(dO), dk, dv,
                              h->d_Pk, h->d_Pv, acc_dk, acc_dv, rope, h->cfg.n_heads, scale);
@@ -2161,8 +2184,8 @@ extern "C" int agpt_attn_bwd(agpt_attn_handle h, const void* q, const void* k, c
   HIP_TRY(hipSetDevice(h->device));
   const float scale = scale_of(h, opts);
   hipStream_t st = opts ? static_cast<hipStream_t>(opts->stream) : nullptr;
-  RopeArgs rope{nullptr, nullptr, 1};
-  if (opts && opts->rope_cos) rope = RopeArgs{opts->rope_cos, opts->rope_sin, opts->rope_seq_len};
+  RopeArgs rope{nullptr, nullptr, 1, 0};
+  if (opts && opts->rope_cos) rope = RopeArgs{opts->rope_cos, opts->rope_sin, opts->rope_seq_len, 0};
   ProfMarks pm;
   if (opts) pm = ProfMarks{opts->prof_events, opts->n_prof_events, st};
   const hipEvent_t ctx_wait = opts ? static_cast<hipEvent_t>(opts->ctx_wait) : nullptr;

@@ -241,6 +241,39 @@ __device__ __forceinline__ bool in_interval(int q, int iv) {
 __device__ __forceinline__ float ld1(const float* p) { return *p; }
 __device__ __forceinline__ float ld1(const bf16_t* p) { return to_f32(*p); }
 
+// The inverse rotations of depths 1..rows in LDS: per depth and 4 dims
+// (two pairs) one float4 of cos, sin, cos, sin, at the clamped position of
+// the depth. Without it (rows 0) the caller's tables are read.
+__host__ __device__ constexpr size_t rope_lds_bytes(int max_depth, int HD) {
+  return static_cast<size_t>(max_depth) * HD * sizeof(float);
+}
+template <int HD, typename RopeT>
+struct RopeTab {
+  const RopeT rope;
+  const float4* tab;
+  // Fills the table; the caller's next barrier publishes it.
+  __device__ __forceinline__ RopeTab(const RopeT& r, unsigned char* lds) : rope(r), tab(reinterpret_cast<const float4*>(lds)) {
+    for (int i = threadIdx.x; i < r.lds_rows * (HD / 4); i += kThreads) {
+      const int o = min(i / (HD / 4), r.seq_len - 1) * HD + 4 * (i % (HD / 4));
+      reinterpret_cast<float4*>(lds)[i] = make_float4(r.cos_t[o], r.sin_t[o], r.cos_t[o + 2], r.sin_t[o + 2]);
+    }
+  }
+  __device__ __forceinline__ explicit operator bool() const { return rope.cos_t != nullptr; }
+  // Dims d0..d0+3 (d0 a multiple of 4) of a head slice of a row at `depth`.
+  __device__ __forceinline__ void inverse(float (&x)[4], int depth, int d0) const {
+    if (rope.lds_rows) {
+      const float4 t = tab[(depth - 1) * (HD / 4) + d0 / 4];
+      const float x0 = x[0], x1 = x[1], x2 = x[2], x3 = x[3];
+      x[0] = x0 * t.x + x1 * t.y;
+      x[1] = -x0 * t.y + x1 * t.x;
+      x[2] = x2 * t.z + x3 * t.w;
+      x[3] = -x2 * t.w + x3 * t.z;
+    } else {
+      agpt_fast::rope_inverse_part<4, HD>(x, rope.cos_t, rope.sin_t, rope_pos(depth, rope.seq_len), d0);
+    }
+  }
+};
+
 // k-th unit of wave w in snake order.
 __device__ __forceinline__ int snake_unit(int k, int w) { return kWaves * k + ((k & 1) ? kWaves - 1 - w : w); }
 
@@ -790,6 +823,7 @@ __global__ __launch_bounds__(kThreads) void bwd_q_kernel(
   extern __shared__ __align__(16) unsigned char dyn[];
   int* ctr = pl.sched + 1;
   if (threadIdx.x == 0) tb.grab = atomicAdd(ctr, 1);
+  const RopeTab<HD, RopeT> rt(rope, dyn + ST::lds_bytes(pl.max_depth));
   ST st(pl, K, V, Q, dO, O, lse, nullptr, H, 0, dyn, tb);
   ChunkLoop<PlanT> cl(pl, ctr, H / HG, uniform(tb.grab));  // the constructor's barrier publishes the claim
   if (cl.t >= cl.ntiles) return;
@@ -902,14 +936,14 @@ __global__ __launch_bounds__(kThreads) void bwd_q_kernel(
       }
       if (q < st.ntile) {
         const int64_t row = static_cast<int64_t>(st.s) + q;
-        const int pos = rope.cos_t ? rope_pos(tb.depth[q], rope.seq_len) : 0;
+        const int dep = tb.depth[q];
 #pragma unroll
         for (int e = 0; e < UH; ++e) {
           const int h = st.hg * HG + h0 + e;
 #pragma unroll
           for (int j = 0; j < MT; ++j) {
             float v[4] = {dq[e][j][0], dq[e][j][1], dq[e][j][2], dq[e][j][3]};
-            if (rope.cos_t) agpt_fast::rope_inverse_part<4, HD>(v, rope.cos_t, rope.sin_t, pos, kBlk * j + 4 * g);
+            if (rt) rt.inverse(v, dep, kBlk * j + 4 * g);
             store_vec<4>(dQ + row * D + h * HD + kBlk * j + 4 * g, v);
           }
           if (g == 0) Dl[row * H + h] = dl[e];
@@ -942,6 +976,7 @@ __global__ __launch_bounds__(kThreads) void bwd_kv_kernel(
   extern __shared__ __align__(16) unsigned char dyn[];
   int* ctr = pl.sched + 2;
   if (threadIdx.x == 0) tb.grab = atomicAdd(ctr, 1);
+  const RopeTab<HD, RopeT> rt(rope, dyn + ST::lds_bytes(pl.max_depth));
   ST st(pl, K, V, Q, dO, nullptr, lse, Dl, H, 0, dyn, tb);
   ChunkLoop<PlanT> cl(pl, ctr, H / HG, uniform(tb.grab));  // the constructor's barrier publishes the claim
   if (cl.t >= cl.ntiles) return;
@@ -1048,7 +1083,7 @@ __global__ __launch_bounds__(kThreads) void bwd_kv_kernel(
         if (r < st.ntile) {
           const int64_t a = static_cast<int64_t>(st.s) + r;
           const bool done = tb.tend[r] <= st.s + st.ntile;
-          const int pos = rope.cos_t ? rope_pos(tb.depth[r], rope.seq_len) : 0;
+          const int dep = tb.depth[r];
 #pragma unroll
           for (int e = 0; e < UH; ++e) {
             const int hd = st.hg * HG + h0 + e;
@@ -1070,7 +1105,7 @@ __global__ __launch_bounds__(kThreads) void bwd_kv_kernel(
 #pragma unroll
                   for (int x = 0; x < 4; ++x) gv[x] += y[x];
                 }
-                if (rope.cos_t) agpt_fast::rope_inverse_part<4, HD>(gk, rope.cos_t, rope.sin_t, pos, d0);
+                if (rt) rt.inverse(gk, dep, d0);
               }
               store_vec<4>(dK + a * D + hd * HD + d0, gk);
               store_vec<4>(dV + a * D + hd * HD + d0, gv);
@@ -1161,6 +1196,7 @@ __global__ __launch_bounds__(kThreads, (kBwdWaves<HD, HG, kCarry>)) void bwd_ker
   extern __shared__ __align__(16) unsigned char dyn[];
   int* ctr = pl.sched + 1;
   if (threadIdx.x == 0) tb.grab = atomicAdd(ctr, 1);
+  const RopeTab<HD, RopeT> rt(rope, dyn + fused_lds_bytes(pl.max_depth, HG, HD, kCarry));
   ST st(pl, K, V, Q, dO, O, lse, nullptr, H, 0, dyn, tb);
   st.dscale = scale;  // dS = P (dP - δ) scale, with V and δ taken times scale
   ChunkLoop<PlanT> cl(pl, ctr, H / HG, uniform(tb.grab));  // the constructor's barrier publishes the claim
@@ -1273,17 +1309,16 @@ __global__ __launch_bounds__(kThreads, (kBwdWaves<HD, HG, kCarry>)) void bwd_ker
         load_vec<KD>(Gs + qr * WS + hoff + KD * g, ga);
         const f4 l2v = *reinterpret_cast<const f4*>(&tb.l2[hh][q0]);
         const f4 dlv = *reinterpret_cast<const f4*>(&tb.dl[hh][q0]);
-        auto columns = [&] {
+        auto columns = [&](const Tin* rows, float (&out)[MT][4]) {
 #pragma unroll
           for (int j = 0; j < MT; ++j)
 #pragma unroll
-            for (int r = 0; r < 4; ++r) {
-              const int row = (q0 + r) * WS + hoff + kBlk * j + c;
-              gcol[j][r] = ld1(Gs + row);
-              qcol[j][r] = ld1(Qs + row);
-            }
+            for (int r = 0; r < 4; ++r) out[j][r] = ld1(rows + (q0 + r) * WS + hoff + kBlk * j + c);
         };
-        if constexpr (MT == 1) columns();
+        if constexpr (MT == 1) {
+          columns(Gs, gcol);
+          columns(Qs, qcol);
+        }
         __builtin_amdgcn_sched_barrier(0);  // (the scheduler would sink them past the S products)
         f4 sv = f4{0.0f, 0.0f, 0.0f, 0.0f}, tv = sv;
 #pragma unroll
@@ -1295,7 +1330,8 @@ __global__ __launch_bounds__(kThreads, (kBwdWaves<HD, HG, kCarry>)) void bwd_ker
         // the products above have read (all at once they spill).
         if constexpr (MT > 1) {
           __builtin_amdgcn_sched_barrier(0);
-          columns();
+          columns(Gs, gcol);
+          columns(Qs, qcol);
         }
         float p[4], ds[4];
 #pragma unroll
@@ -1357,7 +1393,6 @@ __global__ __launch_bounds__(kThreads, (kBwdWaves<HD, HG, kCarry>)) void bwd_ker
         }
       // Final dK/dV of row a at depth dep: + seeds, inverse RoPE of dK.
       auto finish = [&](int64_t a, int dep) {
-        const int pos = rope.cos_t ? rope_pos(dep, rope.seq_len) : 0;
 #pragma unroll
         for (int j = 0; j < MT; ++j) {
           const int d0 = kBlk * j + 4 * g;
@@ -1373,7 +1408,7 @@ __global__ __launch_bounds__(kThreads, (kBwdWaves<HD, HG, kCarry>)) void bwd_ker
 #pragma unroll
             for (int x = 0; x < 4; ++x) gv[j][x] += y[x];
           }
-          if (rope.cos_t) agpt_fast::rope_inverse_part<4, HD>(gk[j], rope.cos_t, rope.sin_t, pos, d0);
+          if (rt) rt.inverse(gk[j], dep, d0);
           store_vec<4>(dK + a * D + hd * HD + d0, gk[j]);
           store_vec<4>(dV + a * D + hd * HD + d0, gv[j]);
         }
@@ -1522,9 +1557,7 @@ __global__ __launch_bounds__(kThreads, (kBwdWaves<HD, HG, kCarry>)) void bwd_ker
 #pragma unroll
           for (int r = 0; r < 4; ++r) qv[x][j][r] = dqr[x][j][r];
           const int q = kBlk * x + c;
-          if (wl == 0 && rope.cos_t && q < nt0)
-            agpt_fast::rope_inverse_part<4, HD>(qv[x][j], rope.cos_t, rope.sin_t, rope_pos(tb.depth[q], rope.seq_len),
-                                                kBlk * j + 4 * g);
+          if (wl == 0 && rt && q < nt0) rt.inverse(qv[x][j], tb.depth[q], kBlk * j + 4 * g);
         }
       more = cl.end_tile(st);
       if (wl == 0)
@@ -1556,8 +1589,7 @@ __global__ __launch_bounds__(kThreads, (kBwdWaves<HD, HG, kCarry>)) void bwd_ker
       for (int w = 1; w < WPH; ++w) sum += *reinterpret_cast<const f4*>(dqs + ((e * WPH + w) * kTile + q) * HD + d0);
 #pragma unroll
       for (int r = 0; r < 4; ++r) qv[k][r] = sum[r];
-      if (rope.cos_t && q < st.ntile)
-        agpt_fast::rope_inverse_part<4, HD>(qv[k], rope.cos_t, rope.sin_t, rope_pos(tb.depth[q], rope.seq_len), d0);
+      if (rt && q < st.ntile) rt.inverse(qv[k], tb.depth[q], d0);
       qo[k] = q < st.ntile ? (static_cast<int64_t>(st.s) + q) * D + (st.hg * HG + e) * HD + d0 : -1;
     }
     more = cl.end_tile(st);

@@ -2,9 +2,11 @@
 (test_gpu_parity's comparison and tolerances)."""
 from __future__ import annotations
 
+import numpy as np
 import pytest
 
-from helpers import small_trie
+from helpers import run_gpu, small_trie, tensors
+from oracle import oracle as ORC
 from test_gpu_parity import _check
 
 pytestmark = pytest.mark.gpu
@@ -23,3 +25,21 @@ def test_path_carry_hd32(gpu, monkeypatch, depth, rows, chunk):
     chunks of one tile and of several, short last tiles."""
     monkeypatch.setenv("AGPT_ATTN_CHUNK", str(chunk))
     _check(_tree(rows, depth, seed=depth), 3, 32, seed=rows, rope=True, acc=True)
+
+
+@pytest.mark.parametrize("hd,dtype,depth,rows", [(16, "f32", 1, 5), (16, "f32", 33, 700), (16, "f32", 72, 900),
+                                                 (32, "f32", 70, 500), (16, "bf16", 33, 700), (32, "bf16", 17, 200)])
+def test_rope_table_in_lds(gpu, monkeypatch, hd, dtype, depth, rows):
+    """The backward's rotations from the table in LDS do the operations of the
+    caller's tables on the same values: the same bytes, and in fp32 the
+    oracle's. Depths past the 64-row tables clamp to their last position."""
+    par = _tree(rows, depth, seed=depth) if depth > 1 else np.full(rows, -1, np.int32)
+    Q, K, V, G = tensors(rows, 2 * hd, rows)
+    res = []
+    for staged in ("0", "1"):
+        monkeypatch.setenv("AGPT_ATTN_ROPELDS", staged)
+        res.append(run_gpu(par, Q, K, V, G, 2, hd, dtype, rope=ORC.rope_table(64, hd)))
+    for name, a, b in zip(("O", "lse", "dQ", "dK", "dV"), *res):
+        np.testing.assert_array_equal(a, b, err_msg=name)
+    if dtype == "f32":
+        _check(par, 2, hd, seed=rows, rope=True)
