@@ -1800,6 +1800,19 @@ void launch_ctx(const agpt_attn_s* h, float* dk, float* dv, RopeArgs rope, hipSt
                      rope, h->cfg.n_heads, h->ctx_add ? 1 : 0);
 }
 
+// Finishes the keys whose carried sums cross chunks. The keys of a chunk go
+// to as many workgroups as bring the grid to ~8 per CU.
+template <int HD>
+void launch_carry(const agpt_attn_s* h, float* dk, float* dv, const float* acc_dk, const float* acc_dv, RopeArgs rope,
+                  hipStream_t st) {
+  const int n = h->n_chunks_sched - 1;
+  if (n < 1) return;
+  const int jobs = agpt_blk::prefix_cap(h->max_depth) * h->cfg.n_heads * HD / 2;
+  const int split = std::max(1, std::min((jobs + agpt_blk::kCarryThreads - 1) / agpt_blk::kCarryThreads, (2048 + n - 1) / n));
+  hipLaunchKernelGGL((agpt_blk::bwd_carry_kernel<HD, PlanDev, RopeArgs>), dim3(n, split), dim3(agpt_blk::kCarryThreads),
+                     0, st, plan_dev(h), h->d_E, h->d_F, dk, dv, acc_dk, acc_dv, rope, h->cfg.n_heads);
+}
+
 template <int HD, typename Tin>
 void launch_bwd(const agpt_attn_s* h, const void* q, const void* k, const void* v, const void* o,
                 const float* lse, const void* dO, float* dq, float* dk, float* dv,
@@ -1837,10 +1850,7 @@ void launch_bwd(const agpt_attn_s* h, const void* q, const void* k, const void* 
       if (h->carry) {
         pm.mark(2);
         pm.mark(3);
-        if (h->n_chunks_sched > 1)
-          hipLaunchKernelGGL((agpt_blk::bwd_carry_kernel<HD, PlanDev, RopeArgs>), dim3(h->n_chunks_sched - 1),
-                             dim3(256), 0, st, plan_dev(h), h->d_E, h->d_F, dk, dv, acc_dk, acc_dv, rope,
-                             h->cfg.n_heads);
+        launch_carry<HD>(h, dk, dv, acc_dk, acc_dv, rope, st);
         launch_ctx<HD>(h, dk, dv, rope, st, ctx_wait);
         pm.mark(4);
         return;
@@ -1942,10 +1952,7 @@ void launch_bwd(const agpt_attn_s* h, const void* q, const void* k, const void* 
                            rope, h->cfg.n_heads, scale);
         pm.mark(2);
         pm.mark(3);
-        if (h->n_chunks_sched > 1)
-          hipLaunchKernelGGL((agpt_blk::bwd_carry_kernel<HD, PlanDev, RopeArgs>), dim3(h->n_chunks_sched - 1),
-                             dim3(256), 0, st, plan_dev(h), h->d_E, h->d_F, dk, dv, acc_dk, acc_dv, rope,
-                             h->cfg.n_heads);
+        launch_carry<HD>(h, dk, dv, acc_dk, acc_dv, rope, st);
         launch_ctx<HD>(h, dk, dv, rope, st, ctx_wait);
         pm.mark(4);
         return;

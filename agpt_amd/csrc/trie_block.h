@@ -1600,60 +1600,77 @@ __global__ __launch_bounds__(kThreads, (kBwdWaves<HD, HG, kCarry>)) void bwd_ker
 }
 
 // ---------------------------------------------------------------------------
-// Carry reduction: one workgroup per chunk C but the last. The keys first
-// seen in chunk C and still open at its end are the prefix entries d of the
-// next chunk's first tile with row >= the chunk's first row; each one's
-// total is F[C][d] + Σ E[C'][d] over the later chunks C' whose first row
-// lies in its subtree (those are exactly the chunks it reaches, and E[C'][d]
-// is its sum over C'), in chunk order; then seeds and inverse RoPE.
-// E, F: [n_chunks][P][2][D] (dK, dV).
+// Carry reduction over the chunks C but the last (blockIdx.x; the keys of a
+// chunk are split over blockIdx.y). The keys first seen in chunk C and still
+// open at its end are the prefix entries d >= d0 of the next chunk's first
+// tile with row >= the chunk's first row; each one's total is F[C][d] +
+// Σ E[C'][d] over the later chunks C' whose first row lies in its subtree
+// (those are exactly the chunks it reaches, and E[C'][d] is its sum over C');
+// then seeds and inverse RoPE. E, F: [n_chunks][P][2][D] (dK, dV).
+//
+// The entries' subtrees are nested, so the long sums (more than kLongSum
+// chunks: a root child can span all of them) are the shallowest ones. They
+// are bound by the latency of their chain of loads: the workgroup's 8 waves
+// each take a contiguous part of the chunks and the parts are added in order.
+// The others, most of the keys, take one thread per 4 columns; blockIdx.y
+// spreads them where there are few chunks. 744K rows of 8 x 64 in 258 chunks:
+// 187 -> 57 us (E and F are 270 MB: 55 us at the copy rate); 242K rows of
+// 4 x 64, depth 160: 149 -> 73 us.
 // ---------------------------------------------------------------------------
+constexpr int kCarryThreads = 512;
+constexpr int kLongSum = 16;
+
+// v += Σ E rows c0 .. c1-1 (cstride floats apart), in order, eight in flight.
+__device__ __forceinline__ void add_chunks(float (&v)[4], const float* __restrict__ e0, int64_t cstride, int c0, int c1) {
+  int c2 = c0;
+  for (; c2 + 8 <= c1; c2 += 8) {
+    float y[8][4];
+#pragma unroll
+    for (int u = 0; u < 8; ++u) load_vec<4>(e0 + (c2 + u) * cstride, y[u]);
+#pragma unroll
+    for (int u = 0; u < 8; ++u)
+#pragma unroll
+      for (int x = 0; x < 4; ++x) v[x] += y[u][x];
+  }
+  for (; c2 < c1; ++c2) {
+    float y[4];
+    load_vec<4>(e0 + c2 * cstride, y);
+#pragma unroll
+    for (int x = 0; x < 4; ++x) v[x] += y[x];
+  }
+}
+
 template <int HD, typename PlanT, typename RopeT>
-__global__ __launch_bounds__(256) void bwd_carry_kernel(PlanT pl, const float* __restrict__ E,
-                                                        const float* __restrict__ F, float* __restrict__ dK,
-                                                        float* __restrict__ dV, const float* __restrict__ acc_dk,
-                                                        const float* __restrict__ acc_dv, RopeT rope, int H) {
+__global__ __launch_bounds__(kCarryThreads) void bwd_carry_kernel(
+    PlanT pl, const float* __restrict__ E, const float* __restrict__ F, float* __restrict__ dK,
+    float* __restrict__ dV, const float* __restrict__ acc_dk, const float* __restrict__ acc_dv, RopeT rope, int H) {
+  constexpr int kParts = kCarryThreads / 64;
+  __shared__ float4 part[kParts][64];
   const int C = blockIdx.x;
   const int K = pl.chunk_tiles;
   const int64_t rows_per_chunk = static_cast<int64_t>(K) * kTile;
   const int64_t sC = C * rows_per_chunk;
   const int t1 = (C + 1) * K;
   const int off = pl.pref_off[t1];
-  const int A = pl.pref_off[t1 + 1] - off;
+  const int A = pl.pref_off[t1 + 1] - off;  // < kMaxDepth <= kCarryThreads
   const int P = prefix_cap(pl.max_depth);
   const int D = H * HD;
   const int Q = D / 2;  // 4-float jobs of a row: dK then dV
-  for (int j = threadIdx.x; j < A * Q; j += blockDim.x) {
-    const int d = j / Q;
-    const int q = j - d * Q;
-    const int64_t a = pl.prefix[off + d];
-    if (a < sC) continue;  // first seen before chunk C: summed by its own chunk's job
+  const int64_t cstride = static_cast<int64_t>(P) * 2 * D;
+  auto c_end = [&](int64_t ea) {
+    return static_cast<int>(min(static_cast<int64_t>(pl.n_chunks), (ea + rows_per_chunk - 1) / rows_per_chunk));
+  };
+  const int tid = threadIdx.x;
+  const bool entry = tid < A;
+  const int64_t ea = entry ? pl.pref_end[off + tid] : 0;
+  const bool own = entry && pl.prefix[off + tid] >= sC;  // else summed by its own chunk's job
+  const int d0 = A - __syncthreads_count(own);
+  const int nlong = __syncthreads_count(own && c_end(ea) - (C + 1) > kLongSum);
+  auto src = [&](const float* base, int64_t c, int d, int q) { return base + c * cstride + static_cast<int64_t>(d) * 2 * D + 4 * q; };
+  auto finish = [&](int d, int q, float (&v)[4]) {
     const int tv = q / (D / 4);
     const int col = (q - tv * (D / 4)) * 4;
-    const int64_t ea = pl.end[a];
-    float v[4];
-    load_vec<4>(F + ((static_cast<int64_t>(C) * P + d) * 2 + tv) * D + col, v);
-    // Chunks c2 > C with c2's first row inside the subtree; eight loads in
-    // flight at a time, added in chunk order.
-    const int c_end = static_cast<int>(min(static_cast<int64_t>(pl.n_chunks), (ea + rows_per_chunk - 1) / rows_per_chunk));
-    const float* e0 = E + (static_cast<int64_t>(d) * 2 + tv) * D + col;
-    const int64_t cstride = static_cast<int64_t>(P) * 2 * D;
-    int c2 = C + 1;
-    for (; c2 + 8 <= c_end; c2 += 8) {
-      float y[8][4];
-#pragma unroll
-      for (int u = 0; u < 8; ++u) load_vec<4>(e0 + (c2 + u) * cstride, y[u]);
-#pragma unroll
-      for (int u = 0; u < 8; ++u)
-#pragma unroll
-        for (int x = 0; x < 4; ++x) v[x] += y[u][x];
-    }
-    for (; c2 < c_end; ++c2) {
-      float y[4];
-      load_vec<4>(e0 + c2 * cstride, y);
-#pragma unroll
-      for (int x = 0; x < 4; ++x) v[x] += y[x];
-    }
+    const int64_t a = pl.prefix[off + d];
     const float* acc = tv ? acc_dv : acc_dk;
     if (acc) {
       float y[4];
@@ -1664,6 +1681,40 @@ __global__ __launch_bounds__(256) void bwd_carry_kernel(PlanT pl, const float* _
     if (tv == 0 && rope.cos_t)
       agpt_fast::rope_inverse_part<4, HD>(v, rope.cos_t, rope.sin_t, rope_pos(d + 1, rope.seq_len), col % HD);
     store_vec<4>((tv ? dV : dK) + a * D + col, v);
+  };
+  // Long sums: (entry, 64 jobs) units.
+  const int nqb = (Q + 63) / 64;
+  const int wave = tid >> 6, lane = tid & 63;
+  for (int u = blockIdx.y; u < nlong * nqb; u += gridDim.y) {
+    const int d = d0 + u / nqb;
+    const int q = (u % nqb) * 64 + lane;
+    const int n = c_end(pl.pref_end[off + d]) - (C + 1);
+    float v[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+    if (q < Q) add_chunks(v, src(E, 0, d, q), cstride, C + 1 + n * wave / kParts, C + 1 + n * (wave + 1) / kParts);
+    part[wave][lane] = make_float4(v[0], v[1], v[2], v[3]);
+    __syncthreads();
+    if (wave == 0 && q < Q) {
+      load_vec<4>(src(F, C, d, q), v);
+#pragma unroll
+      for (int w = 0; w < kParts; ++w) {
+        const float4 y = part[w][lane];
+        v[0] += y.x;
+        v[1] += y.y;
+        v[2] += y.z;
+        v[3] += y.w;
+      }
+      finish(d, q, v);
+    }
+    __syncthreads();
+  }
+  const int jobs = (A - d0 - nlong) * Q;
+  for (int j = blockIdx.y * kCarryThreads + tid; j < jobs; j += gridDim.y * kCarryThreads) {
+    const int d = d0 + nlong + j / Q;
+    const int q = j % Q;
+    float v[4];
+    load_vec<4>(src(F, C, d, q), v);
+    add_chunks(v, src(E, 0, d, q), cstride, C + 1, c_end(pl.pref_end[off + d]));
+    finish(d, q, v);
   }
 }
 

@@ -43,3 +43,15 @@ def test_rope_table_in_lds(gpu, monkeypatch, hd, dtype, depth, rows):
         np.testing.assert_array_equal(a, b, err_msg=name)
     if dtype == "f32":
         _check(par, 2, hd, seed=rows, rope=True)
+
+
+@pytest.mark.parametrize("H,hd,dtype,rows,chunk", [(3, 16, "f32", 17 * 64 + 1, 1), (8, 16, "f32", 30 * 64, 1),
+                                                   (5, 32, "f32", 40 * 64 + 7, 2), (3, 64, "f32", 36 * 64 + 1, 2)])
+def test_carry_sums_over_many_chunks(gpu, monkeypatch, H, hd, dtype, rows, chunk):
+    """One root over every chunk: sums of 16 chunks or fewer (one thread
+    each) and longer ones (split over the workgroup's waves), rows narrower
+    and wider than a wave's 64 column groups."""
+    monkeypatch.setenv("AGPT_ATTN_CHUNK", str(chunk))
+    par = _tree(rows - 1, 20, seed=rows)
+    par = np.concatenate([[-1], par + 1]).astype(np.int32)
+    _check(par, H, hd, seed=rows, dtype=dtype, rope=True, acc=True)
