@@ -251,11 +251,15 @@ template <int HD, typename RopeT>
 struct RopeTab {
   const RopeT rope;
   const float4* tab;
-  // Fills the table; the caller's next barrier publishes it.
-  __device__ __forceinline__ RopeTab(const RopeT& r, unsigned char* lds) : rope(r), tab(reinterpret_cast<const float4*>(lds)) {
-    for (int i = threadIdx.x; i < r.lds_rows * (HD / 4); i += kThreads) {
-      const int o = min(i / (HD / 4), r.seq_len - 1) * HD + 4 * (i % (HD / 4));
-      reinterpret_cast<float4*>(lds)[i] = make_float4(r.cos_t[o], r.sin_t[o], r.cos_t[o + 2], r.sin_t[o + 2]);
+  __device__ __forceinline__ RopeTab(const RopeT& r, unsigned char* lds)
+      : rope(r), tab(reinterpret_cast<const float4*>(lds)) {}
+  // Fills the table (while the first tile's rows are in flight); the
+  // caller's next barrier publishes it.
+  __device__ __forceinline__ void fill() {
+    float4* const t = const_cast<float4*>(tab);
+    for (int i = threadIdx.x; i < rope.lds_rows * (HD / 4); i += kThreads) {
+      const int o = min(i / (HD / 4), rope.seq_len - 1) * HD + 4 * (i % (HD / 4));
+      t[i] = make_float4(rope.cos_t[o], rope.sin_t[o], rope.cos_t[o + 2], rope.sin_t[o + 2]);
     }
   }
   __device__ __forceinline__ explicit operator bool() const { return rope.cos_t != nullptr; }
@@ -341,8 +345,13 @@ struct BStream {
     pdl = reinterpret_cast<float*>(dyn + ((tbytes + 15) & ~15));
     s = 0;
     A = 0;
-    // Every staged value stays finite: a matrix step multiplies dead slots
-    // and rows past the tile by zero weights, and 0 * NaN would leak.
+  }
+
+  // Clears the stream's LDS. Every staged value stays finite: a matrix step
+  // multiplies dead slots and rows past the tile by zero weights, and 0 * NaN
+  // would leak. (After the first prefetch, to overlap it, costs the one-pass
+  // backward 30 VGPRs.)
+  __device__ __forceinline__ void clear(unsigned char* dyn) {
     const int n16 = static_cast<int>(lds_bytes(pl.max_depth) / 16);
     u4* z = reinterpret_cast<u4*>(dyn);
     for (int j = threadIdx.x; j < n16; j += kThreads) z[j] = u4{0u, 0u, 0u, 0u};
@@ -518,14 +527,30 @@ struct BStream {
         }
       }
     } else {
-      for (int j = tid; j < n_A * PJ; j += kThreads) {
-        const int d = j / PJ;
-        const int rem = j % PJ;
-        const int id = pl.prefix[n_poff + d];
-        *reinterpret_cast<u4*>((rem < CPR ? Ks : Vs) + (P - n_A + d) * WS + (rem % CPR) * EPC) =
-            *reinterpret_cast<const u4*>(gsrc(rem < CPR ? K : V, id, rem % CPR));
-        if (rem == 0) set_prefix_entry(d, pl.pref_end[n_poff + d]);
+      // The first kCopyPer rounds take the rows' ids from the prefetch, all
+      // their loads in flight together.
+      auto row = [&](int id, int rem) {
+        return *reinterpret_cast<const u4*>(gsrc(rem < CPR ? K : V, id, rem % CPR));
+      };
+      auto put = [&](int d, int rem, u4 x, int e) {
+        *reinterpret_cast<u4*>((rem < CPR ? Ks : Vs) + (P - n_A + d) * WS + (rem % CPR) * EPC) = x;
+        if (rem == 0) set_prefix_entry(d, e);
+      };
+#pragma unroll
+      for (int k = 0; k < kCopyPer; ++k) {
+        const int d = (tid + k * kThreads) / PJ;
+        if (d < n_A) {
+          cpv[k] = row(cp_id[k], (tid + k * kThreads) % PJ);
+          cpe[k] = pl.pref_end[n_poff + d];
+        }
       }
+#pragma unroll
+      for (int k = 0; k < kCopyPer; ++k) {
+        const int d = (tid + k * kThreads) / PJ;
+        if (d < n_A) put(d, (tid + k * kThreads) % PJ, cpv[k], cpe[k]);
+      }
+      for (int j = tid + kCopyPer * kThreads; j < n_A * PJ; j += kThreads)
+        put(j / PJ, j % PJ, row(pl.prefix[n_poff + j / PJ], j % PJ), pl.pref_end[n_poff + j / PJ]);
     }
     // Dead slots of the first prefix block, and the tile rows.
     const int dead0 = (P - n_A) & ~(kBlk - 1);
@@ -575,10 +600,12 @@ struct BStream {
 };
 
 // ---------------------------------------------------------------------------
-// Dynamic tile chunks. Workgroups claim (chunk, head group) pairs from one
-// counter per kernel (chunk c = tiles [cK, (c+1)K), the last chunk running
-// to the end). A workgroup claims
-// its next chunk during the current one, so with three or more tiles per
+// Dynamic tile chunks. Workgroups claim (chunk, head group) pairs (chunk c =
+// tiles [cK, (c+1)K), the last chunk running to the end): workgroup b starts
+// on claim b, further claims come from one counter per kernel, cleared
+// before the launch, counted on from the grid size. Where the grid covers
+// every claim no counter is read, nor cleared by a launch of its own (see
+// clear_sched_past). A workgroup claims its next chunk during the current one, so with three or more tiles per
 // chunk the claim is known before the last tile's prefetch; within a chunk
 // the prefix moves LDS to LDS, the first tile of a chunk loads it from
 // memory. Results do not depend on which workgroup takes a tile.
@@ -596,8 +623,14 @@ struct ChunkLoop {
   __device__ __forceinline__ int chunk_of(int c) const { return c / ngr; }
   __device__ __forceinline__ bool valid(int c) const { return chunk_of(c) < nch; }
 
-  __device__ __forceinline__ ChunkLoop(const PlanT& pl, int* ctr_, int ngr_, int c)
+  __device__ __forceinline__ ChunkLoop(const PlanT& pl, int* ctr_, int ngr_)
       : ctr(ctr_), nch(pl.n_chunks), ngr(ngr_), K(pl.chunk_tiles), ntiles(pl.n_tiles) {
+    // The block's number through an opaque move: with the claim visible to
+    // the compiler it hoists the tiles' address arithmetic out of the loop
+    // (the one-pass backward 224 -> 253 VGPRs, 28 spilled at head_dim 32).
+    int c = static_cast<int>(blockIdx.x);
+    asm volatile("" : "+v"(c));
+    c = uniform(c);
     hg = c % ngr;
     t = valid(c) ? chunk_of(c) * K : ntiles;
     tend = valid(c) ? cend(chunk_of(c)) : ntiles;
@@ -606,6 +639,11 @@ struct ChunkLoop {
     phase = 0;
     gr = 0;
     sent = known = false;
+  }
+  // The next claim (one lane's; past the last one where the grid covers all).
+  __device__ __forceinline__ int claim() {
+    const int n = static_cast<int>(gridDim.x);
+    return n < nch * ngr ? n + atomicAdd(ctr, 1) : n;
   }
   __device__ __forceinline__ int cend(int ch) const { return ch == nch - 1 ? ntiles : (ch + 1) * K; }
 
@@ -623,7 +661,7 @@ struct ChunkLoop {
   __device__ __forceinline__ void begin_tile(ST& st) {
     const bool within = t + 1 < tend;
     if (!within && !known) {
-      if (!sent && threadIdx.x == 0) gr = atomicAdd(ctr, 1);
+      if (!sent && threadIdx.x == 0) gr = claim();
       sent = true;
       if (threadIdx.x == 0) st.tb.grab = gr;
       __syncthreads();
@@ -641,7 +679,7 @@ struct ChunkLoop {
     if (nt < 0) return false;
     const bool cold = t + 1 >= tend;
     const bool pub = phase == 1 && !known;
-    if (!sent && threadIdx.x == 0) gr = atomicAdd(ctr, 1);
+    if (!sent && threadIdx.x == 0) gr = claim();
     sent = true;
     st.commit(cold, pub, gr);
     if (pub) learn(st);
@@ -677,17 +715,16 @@ __global__ __launch_bounds__(kThreads) void fwd_kernel(PlanT pl, const Tin* __re
   constexpr int WS = ST::WS;
   __shared__ typename ST::Tables tb;
   extern __shared__ __align__(16) unsigned char dyn[];
-  int* ctr = pl.sched + 0;
-  if (threadIdx.x == 0) tb.grab = atomicAdd(ctr, 1);
-  ST st(pl, K, V, Q, nullptr, nullptr, nullptr, nullptr, H, 0, dyn, tb);
-  ChunkLoop<PlanT> cl(pl, ctr, H / HG, uniform(tb.grab));  // the constructor's barrier publishes the claim
+  ChunkLoop<PlanT> cl(pl, pl.sched + 0, H / HG);
   if (cl.t >= cl.ntiles) return;
+  ST st(pl, K, V, Q, nullptr, nullptr, nullptr, nullptr, H, 0, dyn, tb);
   const int lane = threadIdx.x & 63;
   const int wave = threadIdx.x >> 6;
   const int g = lane >> 4, c = lane & 15;
   const int D = H * HD;
   const float qscale = scale * kLog2e;
   const int P = st.P;
+  st.clear(dyn);
   st.prefetch(cl.t, cl.hg);
   st.commit(true);
   do {
@@ -821,12 +858,10 @@ __global__ __launch_bounds__(kThreads) void bwd_q_kernel(
   constexpr int WS = ST::WS;
   __shared__ typename ST::Tables tb;
   extern __shared__ __align__(16) unsigned char dyn[];
-  int* ctr = pl.sched + 1;
-  if (threadIdx.x == 0) tb.grab = atomicAdd(ctr, 1);
-  const RopeTab<HD, RopeT> rt(rope, dyn + ST::lds_bytes(pl.max_depth));
-  ST st(pl, K, V, Q, dO, O, lse, nullptr, H, 0, dyn, tb);
-  ChunkLoop<PlanT> cl(pl, ctr, H / HG, uniform(tb.grab));  // the constructor's barrier publishes the claim
+  ChunkLoop<PlanT> cl(pl, pl.sched + 1, H / HG);
   if (cl.t >= cl.ntiles) return;
+  ST st(pl, K, V, Q, dO, O, lse, nullptr, H, 0, dyn, tb);
+  RopeTab<HD, RopeT> rt(rope, dyn + ST::lds_bytes(pl.max_depth));
   const int lane = threadIdx.x & 63;
   const int wave = threadIdx.x >> 6;
   const int g = lane >> 4, c = lane & 15;
@@ -835,7 +870,9 @@ __global__ __launch_bounds__(kThreads) void bwd_q_kernel(
   const int P = st.P;
   const Tin* Qs = st.Ts;
   const Tin* Gs = st.Ts + kTile * WS;
+  st.clear(dyn);
   st.prefetch(cl.t, cl.hg);
+  rt.fill();
   st.commit(true);
   do {
     cl.begin_tile(st);
@@ -974,12 +1011,10 @@ __global__ __launch_bounds__(kThreads) void bwd_kv_kernel(
   constexpr int WS = ST::WS;
   __shared__ typename ST::Tables tb;
   extern __shared__ __align__(16) unsigned char dyn[];
-  int* ctr = pl.sched + 2;
-  if (threadIdx.x == 0) tb.grab = atomicAdd(ctr, 1);
-  const RopeTab<HD, RopeT> rt(rope, dyn + ST::lds_bytes(pl.max_depth));
-  ST st(pl, K, V, Q, dO, nullptr, lse, Dl, H, 0, dyn, tb);
-  ChunkLoop<PlanT> cl(pl, ctr, H / HG, uniform(tb.grab));  // the constructor's barrier publishes the claim
+  ChunkLoop<PlanT> cl(pl, pl.sched + 2, H / HG);
   if (cl.t >= cl.ntiles) return;
+  ST st(pl, K, V, Q, dO, nullptr, lse, Dl, H, 0, dyn, tb);
+  RopeTab<HD, RopeT> rt(rope, dyn + ST::lds_bytes(pl.max_depth));
   const int lane = threadIdx.x & 63;
   const int wave = threadIdx.x >> 6;
   const int g = lane >> 4, c = lane & 15;
@@ -988,7 +1023,9 @@ __global__ __launch_bounds__(kThreads) void bwd_kv_kernel(
   const int P = st.P;
   const Tin* Qs = st.Ts;
   const Tin* Gs = st.Ts + kTile * WS;
+  st.clear(dyn);
   st.prefetch(cl.t, cl.hg);
+  rt.fill();
   st.commit(true);
   do {
     cl.begin_tile(st);
@@ -1194,13 +1231,11 @@ __global__ __launch_bounds__(kThreads, (kBwdWaves<HD, HG, kCarry>)) void bwd_ker
   constexpr int WS = ST::WS;
   __shared__ typename ST::Tables tb;
   extern __shared__ __align__(16) unsigned char dyn[];
-  int* ctr = pl.sched + 1;
-  if (threadIdx.x == 0) tb.grab = atomicAdd(ctr, 1);
-  const RopeTab<HD, RopeT> rt(rope, dyn + fused_lds_bytes(pl.max_depth, HG, HD, kCarry));
+  ChunkLoop<PlanT> cl(pl, pl.sched + 1, H / HG);
+  if (cl.t >= cl.ntiles) return;
   ST st(pl, K, V, Q, dO, O, lse, nullptr, H, 0, dyn, tb);
   st.dscale = scale;  // dS = P (dP - δ) scale, with V and δ taken times scale
-  ChunkLoop<PlanT> cl(pl, ctr, H / HG, uniform(tb.grab));  // the constructor's barrier publishes the claim
-  if (cl.t >= cl.ntiles) return;
+  RopeTab<HD, RopeT> rt(rope, dyn + fused_lds_bytes(pl.max_depth, HG, HD, kCarry));
   const int lane = threadIdx.x & 63;
   const int wave = threadIdx.x >> 6;
   const int g = lane >> 4, c = lane & 15;
@@ -1221,7 +1256,9 @@ __global__ __launch_bounds__(kThreads, (kBwdWaves<HD, HG, kCarry>)) void bwd_ker
   static_assert(2 * NQB * MT * 64 * 4 <= 2 * kTile * WS, "dQ exchange fits the staged tile");
   const int hh = wave / WPH;  // this wave's head of the group
   const int wl = wave % WPH;  // and its place among that head's waves
+  st.clear(dyn);
   st.prefetch(cl.t, cl.hg);
+  rt.fill();
   st.commit(true);
   bool more;
   do {

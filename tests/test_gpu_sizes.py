@@ -55,3 +55,22 @@ def test_carry_sums_over_many_chunks(gpu, monkeypatch, H, hd, dtype, rows, chunk
     par = _tree(rows - 1, 20, seed=rows)
     par = np.concatenate([[-1], par + 1]).astype(np.int32)
     _check(par, H, hd, seed=rows, dtype=dtype, rope=True, acc=True)
+
+
+@pytest.mark.parametrize("H,hd,dtype", [(4, 16, "f32"), (3, 32, "f32"), (4, 16, "bf16")])
+@pytest.mark.parametrize("chunk", [1, 3])
+def test_more_claims_than_workgroups(gpu, monkeypatch, H, hd, dtype, chunk):
+    """Plans on both sides of one claim per workgroup: a few tiles (no
+    counter is read), and more (chunk, head group) claims than the chip
+    holds workgroups, twice over the same counters, the same bytes."""
+    monkeypatch.setenv("AGPT_ATTN_CHUNK", str(chunk))
+    tr = small_trie(n_tokens=26000, order=4, vocab=30, depth=12, seed=9)
+    for rows in (100, 3 * 2048 * 64 // 2 + 65):
+        par = tr.parent[:rows]
+        assert par.shape[0] == rows
+        Q, K, V, G = tensors(rows, H * hd, 5)
+        a = run_gpu(par, Q, K, V, G, H, hd, dtype)
+        b = run_gpu(par, Q, K, V, G, H, hd, dtype)
+        for name, x, y in zip(("O", "lse", "dQ", "dK", "dV"), a, b):
+            np.testing.assert_array_equal(x, y, err_msg=name)
+    _check(tr.parent[:3000], H, hd, seed=6, dtype="f32")
