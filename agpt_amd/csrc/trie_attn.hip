@@ -1335,19 +1335,29 @@ int plan_impl(agpt_attn_s* h, const int32_t* ext, int64_t n_ext, int32_t A0,
         h->chain_fused = env_int("AGPT_ATTN_CHAINFUSE", 1) != 0;
       }
     }
-    // Up to 24 tiles per claim (the carry's reach), but at least ~8 chunks
-    // per CU: a plan of few tiles (C5: 2048) would otherwise leave most
-    // workgroups without a chunk.
+    // Tiles per claim; claims are (chunk, head group) pairs (heads one by one
+    // on the deep key side). 8 claims per CU; 16 where a tile takes longer
+    // (one-pass head_dim 32, bf16), as the last claims of a launch leave the
+    // other workgroups idle; up to the carry's reach of 24 tiles (96 on the
+    // deep key side). Below that, at least 3 tiles while every workgroup (2
+    // per CU) still gets a claim: each chunk reads its first tile's prefix
+    // from memory and writes E and F rows for the carry kernel. The deep key
+    // side takes 2 at least: chunks of one tile carry nothing and leave
+    // per-tile partials. Without a carry (the split block kernels) long chunks
+    // only save prefix reads: 4 at most. Forward + backward, 8 claims per CU
+    // and no floor against this rule: 31K rows of 8 x 64 bf16, depth 128, 1.67
+    // ms (chunks of 1) -> 0.30 (3); 767K of 4 x 32 1.91 (23) -> 1.69 (11);
+    // 744K of 8 x 64 bf16, depth 128, 3.83 (45) -> 3.68 (22); 90K of 8 x 16
+    // 0.207 (2) -> 0.197 (3); 891K of 8 x 16 bf16 1.59 (13) -> 1.38 (4).
     int cus = 256;
     (void)hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, h->device);
-    // The deep key side's units are (chunk, head): ~8 per CU, and chunks up
-    // to 96 tiles (fewer chunk partials and carry work: C4 83.0 -> 81.6 ms
-    // at 48, the carry kernel 0.70 -> 0.39 ms at 96).
-    // Claims are (chunk, head group) pairs (heads one by one on the deep key side).
-    const int64_t per_claim = static_cast<int64_t>(n_tiles) *
-                              (h->deep_carry ? h->cfg.n_heads : std::max(1, h->cfg.n_heads / std::max(1, h->hg)));
-    const int cap = h->deep_carry ? 96 : 24;
-    const int dflt = static_cast<int>(std::min<int64_t>(cap, std::max<int64_t>(1, per_claim / (8 * std::max(cus, 1)))));
+    cus = std::max(cus, 1);
+    const int64_t claims1 = static_cast<int64_t>(n_tiles) *  // claims of one tile
+                            (h->deep_carry ? h->cfg.n_heads : std::max(1, h->cfg.n_heads / std::max(1, h->hg)));
+    const int64_t cap = h->deep_carry ? 96 : h->carry ? 24 : 4;
+    const int64_t lo = std::max<int64_t>(h->deep_carry ? 2 : 1, std::min<int64_t>(3, claims1 / (2 * cus)));
+    const int per_cu = h->cfg.dtype == AGPT_DTYPE_BF16 || (h->fused && h->cfg.head_dim == 32) ? 16 : 8;
+    const int dflt = static_cast<int>(std::min(cap, std::max(lo, claims1 / (per_cu * cus))));
     h->chunk_tiles = std::max(1, env_int("AGPT_ATTN_CHUNK", dflt));
     h->n_chunks_sched = std::max<int32_t>(1, n_tiles / h->chunk_tiles);
     // Chunks of one tile would carry nothing: the per-tile partials serve.

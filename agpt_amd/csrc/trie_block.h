@@ -1647,12 +1647,12 @@ __global__ __launch_bounds__(kThreads, (kBwdWaves<HD, HG, kCarry>)) void bwd_ker
 //
 // The entries' subtrees are nested, so the long sums (more than kLongSum
 // chunks: a root child can span all of them) are the shallowest ones. They
-// are bound by the latency of their chain of loads: the workgroup's 8 waves
-// each take a contiguous part of the chunks and the parts are added in order.
-// The others, most of the keys, take one thread per 4 columns; blockIdx.y
-// spreads them where there are few chunks. 744K rows of 8 x 64 in 258 chunks:
-// 187 -> 57 us (E and F are 270 MB: 55 us at the copy rate); 242K rows of
-// 4 x 64, depth 160: 149 -> 73 us.
+// are bound by the latency of their loads: the workgroup's 8 waves fetch 32
+// chunks at a time through LDS, the next 32 in flight while one wave adds
+// them in chunk order. The others, most of the keys, take one thread per 4
+// columns; blockIdx.y spreads them where there are few chunks. 744K rows of
+// 8 x 64 in 258 chunks: 187 -> 57 us (E and F are 270 MB: 55 us at the copy
+// rate).
 // ---------------------------------------------------------------------------
 constexpr int kCarryThreads = 512;
 constexpr int kLongSum = 16;
@@ -1681,8 +1681,9 @@ template <int HD, typename PlanT, typename RopeT>
 __global__ __launch_bounds__(kCarryThreads) void bwd_carry_kernel(
     PlanT pl, const float* __restrict__ E, const float* __restrict__ F, float* __restrict__ dK,
     float* __restrict__ dV, const float* __restrict__ acc_dk, const float* __restrict__ acc_dv, RopeT rope, int H) {
-  constexpr int kParts = kCarryThreads / 64;
-  __shared__ float4 part[kParts][64];
+  constexpr int kFetch = 4;                            // chunks a wave fetches per round of a long sum
+  constexpr int kRound = kFetch * kCarryThreads / 64;  // chunks per round
+  __shared__ float4 part[kRound][64];
   const int C = blockIdx.x;
   const int K = pl.chunk_tiles;
   const int64_t rows_per_chunk = static_cast<int64_t>(K) * kTile;
@@ -1725,24 +1726,33 @@ __global__ __launch_bounds__(kCarryThreads) void bwd_carry_kernel(
   for (int u = blockIdx.y; u < nlong * nqb; u += gridDim.y) {
     const int d = d0 + u / nqb;
     const int q = (u % nqb) * 64 + lane;
-    const int n = c_end(pl.pref_end[off + d]) - (C + 1);
-    float v[4] = {0.0f, 0.0f, 0.0f, 0.0f};
-    if (q < Q) add_chunks(v, src(E, 0, d, q), cstride, C + 1 + n * wave / kParts, C + 1 + n * (wave + 1) / kParts);
-    part[wave][lane] = make_float4(v[0], v[1], v[2], v[3]);
-    __syncthreads();
-    if (wave == 0 && q < Q) {
-      load_vec<4>(src(F, C, d, q), v);
+    const int c1 = c_end(pl.pref_end[off + d]);
+    const int qc = min(q, Q - 1);  // lanes past a narrow row repeat its last job
+    float4 y[kFetch];
+    auto fetch = [&](int c) {  // this wave's chunks of the round from chunk c on, clamped
 #pragma unroll
-      for (int w = 0; w < kParts; ++w) {
-        const float4 y = part[w][lane];
-        v[0] += y.x;
-        v[1] += y.y;
-        v[2] += y.z;
-        v[3] += y.w;
-      }
-      finish(d, q, v);
+      for (int x = 0; x < kFetch; ++x)
+        y[x] = *reinterpret_cast<const float4*>(src(E, min(c + wave * kFetch + x, c1 - 1), d, qc));
+    };
+    float v[4];
+    load_vec<4>(src(F, C, d, qc), v);
+    fetch(C + 1);
+    for (int c = C + 1; c < c1; c += kRound) {
+#pragma unroll
+      for (int x = 0; x < kFetch; ++x) part[wave * kFetch + x][lane] = y[x];
+      __syncthreads();
+      if (c + kRound < c1) fetch(c + kRound);
+      if (wave == 0)
+        for (int x = 0; x < min(kRound, c1 - c); ++x) {
+          const float4 e = part[x][lane];
+          v[0] += e.x;
+          v[1] += e.y;
+          v[2] += e.z;
+          v[3] += e.w;
+        }
+      __syncthreads();
     }
-    __syncthreads();
+    if (wave == 0 && q < Q) finish(d, q, v);
   }
   const int jobs = (A - d0 - nlong) * Q;
   for (int j = blockIdx.y * kCarryThreads + tid; j < jobs; j += gridDim.y * kCarryThreads) {

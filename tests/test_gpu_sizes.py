@@ -74,3 +74,13 @@ def test_more_claims_than_workgroups(gpu, monkeypatch, H, hd, dtype, chunk):
         for name, x, y in zip(("O", "lse", "dQ", "dK", "dV"), a, b):
             np.testing.assert_array_equal(x, y, err_msg=name)
     _check(tr.parent[:3000], H, hd, seed=6, dtype="f32")
+
+
+@pytest.mark.parametrize("H,hd,dtype,rows", [(8, 64, "f32", 65), (8, 64, "f32", 128 * 64 + 1), (2, 32, "f32", 300 * 64),
+                                             (8, 16, "f32", 2 * 256 * 64 - 1), (8, 16, "f32", 300 * 64)])
+def test_default_chunk_lengths(gpu, H, hd, dtype, rows):
+    """Plans around the rule's lines: the deep key side's floor of two tiles,
+    fewer claims than workgroups, one claim each, the three-tile floor."""
+    tr = small_trie(n_tokens=26000, order=4, vocab=30, depth=12, seed=9)
+    assert tr.n_nodes >= rows
+    _check(tr.parent[:rows], H, hd, seed=rows, dtype=dtype, rope=True)
