@@ -373,6 +373,17 @@ __global__ __launch_bounds__(64) void varlen_L_bwd_kernel(
 // is the D layout, so a product's registers feed the next one directly.
 constexpr int kLqMaxDelta = 1024;  // queries per node in the backward's per-wave δ table (LDS)
 
+__device__ __forceinline__ int lq_uniform(int v) { return __builtin_amdgcn_readfirstlane(v); }
+
+// Element idx from a wave-uniform base as a 32-bit byte offset (a scalar base
+// and one register per address; a node's rows and weights span < 4 GiB).
+__device__ __forceinline__ const float* lq_at(const float* base, uint32_t idx) {
+  return reinterpret_cast<const float*>(reinterpret_cast<const char*>(base) + idx * 4u);
+}
+__device__ __forceinline__ float* lq_at(float* base, uint32_t idx) {
+  return reinterpret_cast<float*>(reinterpret_cast<char*>(base) + idx * 4u);
+}
+
 // Bit mask of the lanes whose query t = base + lane is its radix node's first.
 __device__ __forceinline__ uint64_t node_starts(const int* __restrict__ q2n, const int* __restrict__ qoff,
                                                 int64_t base, int T_q) {
@@ -437,6 +448,9 @@ constexpr int kLqCache = 4;
 // blocks takes each query's maximum and sum (S^T blocks: query c in lane
 // column c, rows in registers), a second recomputes S^T, writes the
 // normalized weights (visible entries only) and adds O^T += V^T P^T.
+// Bound by the latency of each node's chain of loads, hence by the waves in
+// flight: the loops stay rolled and the addresses are a scalar base with a
+// 32-bit offset, 76 VGPRs for 138 (8 x 16, 1.76M queries: 2.08 -> 1.76 ms).
 template <int HD>
 __global__ __launch_bounds__(256) void varlen_Lq_fwd_kernel(
     const float* __restrict__ q, const float* __restrict__ k, const float* __restrict__ v,
@@ -445,7 +459,7 @@ __global__ __launch_bounds__(256) void varlen_Lq_fwd_kernel(
     int max_len, float scale) {
   constexpr int MT = HD / 16;
   // wave = (block of 64 queries, head)
-  const int64_t wid = static_cast<int64_t>(blockIdx.x) * (blockDim.x >> 6) + (threadIdx.x >> 6);
+  const int64_t wid = static_cast<int64_t>(blockIdx.x) * (blockDim.x >> 6) + lq_uniform(threadIdx.x >> 6);
   const int64_t base = wid / H * 64;
   const int h = static_cast<int>(wid - wid / H * H);
   if (base >= T_q) return;  // uniform per wave
@@ -459,29 +473,33 @@ __global__ __launch_bounds__(256) void varlen_Lq_fwd_kernel(
   while (starts) {
     const int64_t t0 = base + __builtin_ctzll(starts);
     starts &= starts - 1;
-    const int node = q2n[t0];
-    const int L = qoff[node + 1] - static_cast<int>(t0);
-    const int len = min(kv_len[node], max_len);
+    // Wave-uniform values, kept in scalar registers (as do the row pointers
+    // and loop bounds made of them).
+    const int node = lq_uniform(q2n[t0]);
+    const int L = lq_uniform(qoff[node + 1]) - static_cast<int>(t0);
+    const int len = min(lq_uniform(kv_len[node]), max_len);
     if (L < 1 || L > max_len || len < 1) continue;  // inconsistent tables
-    const int64_t off = kv_off[node];
+    const int64_t off = lq_uniform(kv_off[node]);
     const float* qh = q + (t0 * H + h) * HD;  // query j of the node at qh + j RS
     float* oh = out + (t0 * H + h) * HD;
     float* wh = weights + (t0 * H + h) * max_len;
     const float* kh = k + (off * H + h) * HD;  // packed row p at kh + p RS
     const float* vh = v + (off * H + h) * HD;
     const int shift = len - L;  // query j sees rows p <= shift + j
+#pragma unroll 1
     for (int i = 0; i < L; i += 16) {
       const int jq = i + c;  // this lane's query (column)
       const bool qok = jq < L;
       float qy[HD / 4];
-      load_vec<HD / 4>(qh + (qok ? jq : 0) * RS + (HD / 4) * g, qy);
+      load_vec<HD / 4>(lq_at(qh, (qok ? jq : 0) * RS + (HD / 4) * g), qy);
       const int pend = min(len, shift + i + 16);  // rows any query of the block sees
       float m = -INFINITY, l = 0.0f;
       f4 sc[kLqCache];
 #pragma unroll
       for (int x = 0; x < kLqCache; ++x) sc[x] = f4{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll 1
       for (int b = 0; b < pend; b += 16) {
-        const f4 sv0 = lq_rows_dot<HD>(kh + min(b + c, len - 1) * RS, qy, g);
+        const f4 sv0 = lq_rows_dot<HD>(lq_at(kh, min(b + c, len - 1) * RS), qy, g);
 #pragma unroll
         for (int x = 0; x < kLqCache; ++x)
           if (b == 16 * x) sc[x] = sv0;
@@ -503,19 +521,20 @@ __global__ __launch_bounds__(256) void varlen_Lq_fwd_kernel(
       f4 o[MT];
 #pragma unroll
       for (int t = 0; t < MT; ++t) o[t] = f4{0.0f, 0.0f, 0.0f, 0.0f};
-      float* wrow = wh + static_cast<int64_t>(qok ? jq : 0) * WS;
+      float* wrow = lq_at(wh, static_cast<uint32_t>(qok ? jq : 0) * WS);
+#pragma unroll 1
       for (int b = 0; b < pend; b += 16) {
         // V^T operand first: lane (g, c) supplies V[row b + 4g + j][dim 16t + c]
         float vt[MT][4];
 #pragma unroll
         for (int j = 0; j < 4; ++j)
 #pragma unroll
-          for (int t = 0; t < MT; ++t) vt[t][j] = vh[min(b + 4 * g + j, len - 1) * RS + 16 * t + c];
+          for (int t = 0; t < MT; ++t) vt[t][j] = *lq_at(vh, min(b + 4 * g + j, len - 1) * RS + 16 * t + c);
         f4 sv = sc[0];
 #pragma unroll
         for (int x = 1; x < kLqCache; ++x)
           if (b == 16 * x) sv = sc[x];
-        if (b >= 16 * kLqCache) sv = lq_rows_dot<HD>(kh + min(b + c, len - 1) * RS, qy, g);
+        if (b >= 16 * kLqCache) sv = lq_rows_dot<HD>(lq_at(kh, min(b + c, len - 1) * RS), qy, g);
         float pw[4];
         const int vis = qok ? min(len, shift + jq + 1) : 0;  // this query's visible rows
 #pragma unroll
@@ -535,7 +554,7 @@ __global__ __launch_bounds__(256) void varlen_Lq_fwd_kernel(
       // O^T[dim 16t + 4g + r][query c]
       if (qok)
 #pragma unroll
-        for (int t = 0; t < MT; ++t) *reinterpret_cast<f4*>(oh + jq * RS + 16 * t + 4 * g) = o[t];
+        for (int t = 0; t < MT; ++t) *reinterpret_cast<f4*>(lq_at(oh, jq * RS + 16 * t + 4 * g)) = o[t];
     }
   }
 }
@@ -561,7 +580,7 @@ __global__ __launch_bounds__(256) void varlen_Lq_bwd_kernel(
   extern __shared__ double lq_delta[];
   double* delta = lq_delta + (threadIdx.x >> 6) * max_len;
   // wave = (block of 64 queries, head)
-  const int64_t wid = static_cast<int64_t>(blockIdx.x) * (blockDim.x >> 6) + (threadIdx.x >> 6);
+  const int64_t wid = static_cast<int64_t>(blockIdx.x) * (blockDim.x >> 6) + lq_uniform(threadIdx.x >> 6);
   const int64_t base = wid / H * 64;
   const int h = static_cast<int>(wid - wid / H * H);
   if (base >= T_q) return;  // uniform per wave
@@ -575,11 +594,11 @@ __global__ __launch_bounds__(256) void varlen_Lq_bwd_kernel(
   while (starts) {
     const int64_t t0 = base + __builtin_ctzll(starts);
     starts &= starts - 1;
-    const int node = q2n[t0];
-    const int L = qoff[node + 1] - static_cast<int>(t0);
-    const int len = min(kv_len[node], max_len);
+    const int node = lq_uniform(q2n[t0]);
+    const int L = lq_uniform(qoff[node + 1]) - static_cast<int>(t0);
+    const int len = min(lq_uniform(kv_len[node]), max_len);
     if (L < 1 || L > max_len || len < 1) continue;  // inconsistent tables: δ holds max_len queries
-    const int64_t off = kv_off[node];
+    const int64_t off = lq_uniform(kv_off[node]);
     const float* qh = q + (t0 * H + h) * HD;  // query j of the node at + j RS
     const float* gh = d_out + (t0 * H + h) * HD;
     float* dqh = dq + (t0 * H + h) * HD;
@@ -692,6 +711,158 @@ __global__ __launch_bounds__(256) void varlen_Lq_bwd_kernel(
     }
     // the next node's query side rewrites the δ table
     __builtin_amdgcn_wave_barrier();
+  }
+}
+
+// Backward for rows of at most 16 NB keys (max_len <= 16 NB), the same sums
+// in the same order in one pass over a node's query blocks: dW of a query
+// block against every row block is formed once and kept in registers with
+// the weights until δ is known; dS and P go through a per-wave LDS tile into
+// the key side's orientation (write query c's four rows, read row c's four
+// queries; LDS operations of a wave complete in order), and dK, dV of every
+// row block stay in registers over the query blocks. The two-sided kernel
+// above reads V three times and Q, dO, the weights twice, from lines that
+// the other waves in flight have pushed out of L2 by then: 12.8 GB read for
+// 7.7 algorithmic (1.76M queries, 8 x 16): 3.59 -> 2.83 ms; 596K queries of
+// 4 x 32 1.06 -> 0.84 (rows to 32), 2.69 -> 2.29 (rows to 64), of 4 x 64 2.10
+// -> 1.66, of 8 x 16 with rows to 64 3.33 -> 3.17. Two heads per wave (whole
+// lines) in the two-sided kernel ran slower (3.78, 4 waves per SIMD for 5).
+template <int HD, int NB>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(HD * NB == 32 ? 4 : 2))) void varlen_Lq_bwd_short_kernel(
+    const float* __restrict__ q, const float* __restrict__ k, const float* __restrict__ v,
+    const float* __restrict__ weights, const float* __restrict__ d_out, const int* __restrict__ q2n,
+    const int* __restrict__ qoff, const int* __restrict__ kv_off, const int* __restrict__ kv_len,
+    float* __restrict__ dq, float* __restrict__ dk, float* __restrict__ dv, int T_q, int H, int max_len,
+    float scale) {
+  constexpr int MT = HD / 16;
+  constexpr int TS = 20;  // row stride of the 16x16 tiles
+  __shared__ float tiles[4][2][16 * TS];
+  const int wave = lq_uniform(threadIdx.x >> 6);
+  float* pt = tiles[wave][0];
+  float* st = tiles[wave][1];
+  // wave = (block of 64 queries, head)
+  const int64_t wid = static_cast<int64_t>(blockIdx.x) * (blockDim.x >> 6) + wave;
+  const int64_t base = wid / H * 64;
+  const int h = static_cast<int>(wid - wid / H * H);
+  if (base >= T_q) return;  // uniform per wave
+  const int lane = threadIdx.x & 63;
+  const int g = lane >> 4, c = lane & 15;
+  uint64_t starts = node_starts(q2n, qoff, base, T_q);
+  const double dscale = static_cast<double>(scale);
+  const int RS = H * HD;       // row stride of q / k / v / d_out / dq / dk / dv
+  const int WS = H * max_len;  // query stride of the weights
+  const bool wvec = (max_len & 3) == 0;  // weight rows 16-byte aligned
+  while (starts) {
+    const int64_t t0 = base + __builtin_ctzll(starts);
+    starts &= starts - 1;
+    const int node = lq_uniform(q2n[t0]);
+    const int L = lq_uniform(qoff[node + 1]) - static_cast<int>(t0);
+    const int len = min(lq_uniform(kv_len[node]), max_len);
+    if (L < 1 || L > max_len || len < 1) continue;  // inconsistent tables
+    const int64_t off = lq_uniform(kv_off[node]);
+    const float* qh = q + (t0 * H + h) * HD;  // query j of the node at + j RS
+    const float* gh = d_out + (t0 * H + h) * HD;
+    float* dqh = dq + (t0 * H + h) * HD;
+    const float* wh = weights + (t0 * H + h) * max_len;
+    const float* kh = k + (off * H + h) * HD;  // packed row p at + p RS
+    const float* vh = v + (off * H + h) * HD;
+    const int shift = len - L;
+    f4 dka[NB][MT], dva[NB][MT];
+#pragma unroll
+    for (int b = 0; b < NB; ++b)
+#pragma unroll
+      for (int t = 0; t < MT; ++t) {
+        dka[b][t] = f4{0.0f, 0.0f, 0.0f, 0.0f};
+        dva[b][t] = dka[b][t];
+      }
+#pragma unroll 1
+    for (int i = 0; i < L; i += 16) {
+      const int jq = i + c;
+      const bool qok = jq < L;
+      float gy[HD / 4];
+      load_vec<HD / 4>(lq_at(gh, (qok ? jq : 0) * RS + (HD / 4) * g), gy);
+      const float* wrow = lq_at(wh, static_cast<uint32_t>(qok ? jq : 0) * WS);
+      const int vis = qok ? min(len, shift + jq + 1) : 0;  // this query's visible rows
+      const int pend = min(len, shift + i + 16);
+      double dot = 0.0;
+      f4 dw[NB];
+      float wp[NB][4];
+#pragma unroll
+      for (int b = 0; b < NB; ++b) {
+        if (16 * b >= pend) break;
+        dw[b] = lq_rows_dot<HD>(lq_at(vh, min(16 * b + c, len - 1) * RS), gy, g);
+        lq_weights4(wrow, 16 * b + 4 * g, wvec, vis, wp[b]);
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+          if (16 * b + 4 * g + r < vis) dot += static_cast<double>(dw[b][r] * wp[b][r]);
+      }
+      dot = lq_gsum_d(dot);
+      // dO^T, Q^T operands: lane (g, c) supplies row i + 4g + j at dim 16t + c
+      float gt[MT][4], qt[MT][4];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const int jc = min(i + 4 * g + j, L - 1);
+#pragma unroll
+        for (int t = 0; t < MT; ++t) {
+          gt[t][j] = *lq_at(gh, jc * RS + 16 * t + c);
+          qt[t][j] = *lq_at(qh, jc * RS + 16 * t + c);
+        }
+      }
+      f4 dqa[MT];
+#pragma unroll
+      for (int t = 0; t < MT; ++t) dqa[t] = f4{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+      for (int b = 0; b < NB; ++b) {
+        if (16 * b >= pend) break;
+        // K^T operand: lane (g, c) supplies K[row 16b + 4g + j][dim 16t + c]
+        float kt[MT][4];
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+#pragma unroll
+          for (int t = 0; t < MT; ++t) kt[t][j] = *lq_at(kh, min(16 * b + 4 * g + j, len - 1) * RS + 16 * t + c);
+        float ds[4];
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+          ds[r] = static_cast<float>(static_cast<double>(wp[b][r]) * (static_cast<double>(dw[b][r]) - dot) * dscale);
+        *reinterpret_cast<f4*>(pt + c * TS + 4 * g) = f4{wp[b][0], wp[b][1], wp[b][2], wp[b][3]};
+        *reinterpret_cast<f4*>(st + c * TS + 4 * g) = f4{ds[0], ds[1], ds[2], ds[3]};
+#pragma unroll
+        for (int t = 0; t < MT; ++t)
+#pragma unroll
+          for (int j = 0; j < 4; ++j) dqa[t] = lq_mfma(kt[t][j], ds[j], dqa[t]);
+        float wv[4], dsv[4];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          wv[j] = pt[(4 * g + j) * TS + c];
+          dsv[j] = st[(4 * g + j) * TS + c];
+        }
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+#pragma unroll
+          for (int t = 0; t < MT; ++t) {
+            dva[b][t] = lq_mfma(gt[t][j], wv[j], dva[b][t]);
+            dka[b][t] = lq_mfma(qt[t][j], dsv[j], dka[b][t]);
+          }
+      }
+      if (qok)
+#pragma unroll
+        for (int t = 0; t < MT; ++t) *reinterpret_cast<f4*>(lq_at(dqh, jq * RS + 16 * t + 4 * g)) = dqa[t];
+    }
+    // dK^T[dim 16t + 4g + r][row 16b + c]: add into the caller's rows
+    float* dkh = dk + (off * H + h) * HD;
+    float* dvh = dv + (off * H + h) * HD;
+#pragma unroll
+    for (int b = 0; b < NB; ++b) {
+      const int p = 16 * b + c;
+      if (p < len)
+#pragma unroll
+        for (int t = 0; t < MT; ++t) {
+          f4* pk = reinterpret_cast<f4*>(lq_at(dkh, p * RS + 16 * t + 4 * g));
+          f4* pv = reinterpret_cast<f4*>(lq_at(dvh, p * RS + 16 * t + 4 * g));
+          *pk = *pk + dka[b][t];
+          *pv = *pv + dva[b][t];
+        }
+    }
   }
 }
 
@@ -813,10 +984,18 @@ extern "C" int agpt_varlen_attention_L_queries_backward(
     constexpr int HD = decltype(c)::value;
     if (HD % 16 == 0 && max_kv_len <= kLqMaxDelta) {
       const int64_t waves = (static_cast<int64_t>(T_q) + 63) / 64 * n_heads;  // (block of 64 queries, head)
-      hipLaunchKernelGGL((varlen_Lq_bwd_kernel<HD % 16 == 0 ? HD : 16>), dim3(static_cast<unsigned>((waves + 3) / 4)),
-                         dim3(256), sizeof(double) * 4 * max_kv_len, static_cast<hipStream_t>(stream), q, k, v,
-                         attn_weights, d_out, query_to_node, query_offsets, kv_offsets, kv_lengths, dq, dk_full,
-                         dv_full, T_q, n_heads, max_kv_len, scale);
+      auto run = [&](auto fn, size_t lds) {
+        hipLaunchKernelGGL(fn, dim3(static_cast<unsigned>((waves + 3) / 4)), dim3(256), lds,
+                           static_cast<hipStream_t>(stream), q, k, v, attn_weights, d_out, query_to_node,
+                           query_offsets, kv_offsets, kv_lengths, dq, dk_full, dv_full, T_q, n_heads, max_kv_len,
+                           scale);
+      };
+      // Up to 32 or 64 keys the one-pass kernel (its row blocks' sums fit in
+      // registers; at head_dim 64 up to 32).
+      constexpr int HB = HD % 16 == 0 ? HD : 16;
+      if (max_kv_len <= 32) run(varlen_Lq_bwd_short_kernel<HB, 2>, 0);
+      else if (max_kv_len <= 64 && HB <= 32) run(varlen_Lq_bwd_short_kernel<HB, HB <= 32 ? 4 : 2>, 0);
+      else run(varlen_Lq_bwd_kernel<HB>, sizeof(double) * 4 * max_kv_len);
     } else {  // head dims 4 and 8, or a δ table past the wave's LDS share: a workgroup per (radix node, head)
       hipLaunchKernelGGL((varlen_L_bwd_kernel<HD>), dim3(T_q, n_heads), dim3(64),
                          sizeof(double) * max_kv_len, static_cast<hipStream_t>(stream), q, k, v,

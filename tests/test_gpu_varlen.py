@@ -150,3 +150,37 @@ def test_varlen_L_queries(gpu, H, hd, kind):
     assert_close(dq.cpu().numpy(), dq_r, what="L dQ")
     assert_close(dk.cpu().numpy(), dk_r, what="L dK")
     assert_close(dv.cpu().numpy(), dv_r, what="L dV")
+
+
+@pytest.mark.parametrize("H,hd,longest", [(3, 16, 16), (2, 16, 32), (3, 16, 33), (1, 32, 64), (2, 16, 65), (2, 64, 31),
+                                          (1, 64, 33)])
+def test_varlen_L_queries_row_limits(gpu, H, hd, longest):
+    """The backward on both sides of its row limits (32 and 64 keys in one
+    pass, more in two): one node of `longest` rows whose queries are its last
+    1, 17 or all rows, and short nodes around it; dK/dV add into the caller's
+    values."""
+    import torch
+
+    from agpt_amd import attention as A
+    rng = np.random.default_rng(longest)
+    kv_len = np.array([1, longest, longest, longest, 5, 16], np.int32)
+    L = np.array([1, 1, min(17, longest), longest, 3, 16], np.int32)
+    qoff = np.concatenate([[0], np.cumsum(L)]).astype(np.int32)
+    q2n = np.repeat(np.arange(6, dtype=np.int32), L)
+    kv_off = np.concatenate([[0], np.cumsum(kv_len)[:-1]]).astype(np.int32)
+    T, R, D, scale = int(qoff[-1]), int(kv_len.sum()), H * hd, scale_of(hd)
+    Q, G = (rng.standard_normal((T, D)).astype(np.float32) for _ in range(2))
+    K, V, S = (rng.standard_normal((R, D)).astype(np.float32) for _ in range(3))
+    cu = lambda x: torch.from_numpy(np.ascontiguousarray(x)).cuda()
+    tabs = [cu(x) for x in (q2n, qoff, kv_off, kv_len)]
+    out, w = torch.zeros(T * D, device="cuda"), torch.zeros(T * H * longest, device="cuda")
+    A.batched_varlen_attention_L_queries(cu(Q), cu(K), cu(V), *tabs, out, w, T, H, hd, longest, scale)
+    o_ref, w_ref = ORC.varlen_L_fwd(Q, K, V, q2n, qoff, kv_off, kv_len, T, H, hd, longest, scale)
+    assert_close(out.cpu().numpy(), o_ref, what="L O")
+    dq, dk, dv = torch.zeros(T * D, device="cuda"), cu(S.ravel().copy()), cu(S.ravel().copy())
+    A.batched_varlen_attention_L_queries_backward(cu(Q), cu(K), cu(V), w, cu(G), *tabs, dq, dk, dv, T, H, hd, longest,
+                                                  scale)
+    want = ORC.varlen_L_bwd(Q, K, V, w_ref, G, q2n, qoff, kv_off, kv_len, T, H, hd, longest, scale, R,
+                            dk=S.ravel(), dv=S.ravel())
+    for name, got, ref in zip(("dQ", "dK", "dV"), (dq, dk, dv), want):
+        assert_close(got.cpu().numpy(), ref, what=name)
