@@ -1745,6 +1745,20 @@ void with_block_heads(const agpt_attn_s* h, int uh, Fn&& fn) {
   });
 }
 
+// Deep kernels: puts the rotations of every depth in `fn`'s LDS (see
+// choose_variant) when that keeps its workgroups per CU; returns the bytes.
+// 596K rows of 4 x 64, depth 32, with the carry kernel's two turns: fp32 dQ
+// kernel 1.01 -> 0.89 ms, key side 1.62 -> 1.51; bf16 key side 1.01 -> 0.73.
+template <typename Fn>
+size_t stage_rope(const agpt_attn_s* h, Fn fn, size_t lds, int hd, RopeArgs& rope) {
+  const size_t extra = agpt_blk::rope_lds_bytes(h->max_depth, hd);
+  if (!rope.cos_t || env_int("AGPT_ATTN_ROPELDS", 1) == 0) return 0;
+  set_lds(fn, lds + extra);
+  if (wg_per_cu(fn, lds + extra, h->max_lds) < std::max(1, wg_per_cu(fn, lds, h->max_lds))) return 0;
+  rope.lds_rows = h->max_depth;
+  return extra;
+}
+
 template <int HD, typename Tin>
 void launch_fwd(const agpt_attn_s* h, const void* q, const void* k, const void* v, void* o,
                 float* lse, float scale, hipStream_t st, const ProfMarks& pm) {
@@ -1920,10 +1934,12 @@ void launch_bwd(const agpt_attn_s* h, const void* q, const void* k, const void* 
       const int hpu = deep_heads_per_unit(h);
       auto launch_q = [&](auto fq) {
         set_lds(fq, h->bq_lds);
-        hipLaunchKernelGGL(fq, dim3(stream_grid(h, fq, h->bq_lds, hpu)), dim3(agpt_deep::kThreads), h->bq_lds, st,
+        RopeArgs rope_q = rope;
+        const size_t lds = h->bq_lds + (sizeof(Tin) == 4 ? stage_rope(h, fq, h->bq_lds, HD, rope_q) : 0);
+        hipLaunchKernelGGL(fq, dim3(stream_grid(h, fq, lds, hpu)), dim3(agpt_deep::kThreads), lds, st,
                            plan_dev(h), static_cast<const Tin*>(q), static_cast<const Tin*>(k),
                            static_cast<const Tin*>(v), static_cast<const Tin*>(o), lse,
-                           static_cast<const Tin*>(dO), dq, h->d_Dl, rope, h->cfg.n_heads, hpu, scale);
+                           static_cast<const Tin*>(dO), dq, h->d_Dl, rope_q, h->cfg.n_heads, hpu, scale);
       };
       // bf16: δ and dQ in one pass over the key chunks (AGPT_ATTN_DQ1=0: a δ pass, then dQ)
       if constexpr (sizeof(Tin) == 2) {
@@ -1952,18 +1968,23 @@ void launch_bwd(const agpt_attn_s* h, const void* q, const void* k, const void* 
       }
       if (h->deep_carry) {
         // Key slots of a tile: prefix_cap + 64. A plan to depth 128 keeps
-        // every slot's sums in registers (4 kRegIters blocks of 16) and, in
-        // bf16, each slot's K/V slices in an LDS cache tagged by row;
-        // deeper plans (or AGPT_ATTN_REGITERS=2) keep the first 4
-        // kRegItersDeep blocks in registers and the rest in the carry rows.
+        // every slot's sums in registers (2 turns of 4 blocks of 16 to depth
+        // 65, else 3) and, in bf16, each slot's K/V slices in an LDS cache
+        // tagged by row; deeper plans (or AGPT_ATTN_REGITERS=2) keep the first
+        // 4 kRegItersDeep blocks in registers and the rest in the carry rows.
         const bool regs = env_int("AGPT_ATTN_REGCARRY", 1) != 0;
-        const bool all_regs = agpt_blk::prefix_cap(h->max_depth) + agpt_deep::kTile <= 64 * agpt_deep::kRegIters &&
-                              env_int("AGPT_ATTN_REGITERS", agpt_deep::kRegIters) == agpt_deep::kRegIters;
-        auto fc = !regs      ? agpt_deep::bwd_kv_carry_kernel<HD, Tin, 0, PlanDev, RopeArgs>
-                  : all_regs ? agpt_deep::bwd_kv_carry_kernel<HD, Tin, agpt_deep::kRegIters, PlanDev, RopeArgs>
-                             : agpt_deep::bwd_kv_carry_kernel<HD, Tin, agpt_deep::kRegItersDeep, PlanDev, RopeArgs>;
-        const size_t lds =
-            h->kv_lds + agpt_deep::kv_cache_bytes(regs && all_regs ? agpt_deep::kRegIters : 0, sizeof(Tin));
+        const int slots = agpt_blk::prefix_cap(h->max_depth) + agpt_deep::kTile;
+        const int iters = env_int("AGPT_ATTN_REGITERS", 0);  // 0: by depth
+        const bool all2 = slots <= 64 * agpt_deep::kRegItersDeep && iters == 0;
+        const bool all3 = slots <= 64 * agpt_deep::kRegIters && !all2 && (iters == 0 || iters == agpt_deep::kRegIters);
+        auto fc = !regs  ? agpt_deep::bwd_kv_carry_kernel<HD, Tin, 0, false, PlanDev, RopeArgs>
+                  : all2 ? agpt_deep::bwd_kv_carry_kernel<HD, Tin, agpt_deep::kRegItersDeep, true, PlanDev, RopeArgs>
+                  : all3 ? agpt_deep::bwd_kv_carry_kernel<HD, Tin, agpt_deep::kRegIters, true, PlanDev, RopeArgs>
+                         : agpt_deep::bwd_kv_carry_kernel<HD, Tin, agpt_deep::kRegItersDeep, false, PlanDev, RopeArgs>;
+        size_t lds = h->kv_lds + agpt_deep::kv_cache_bytes(all2 ? agpt_deep::kRegItersDeep : agpt_deep::kRegIters,
+                                                           regs && (all2 || all3), sizeof(Tin));
+        RopeArgs rope_kv = rope;
+        lds += stage_rope(h, fc, lds, HD, rope_kv);
         set_lds(fc, lds);
         int cus = 256;
         (void)hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, h->device);
@@ -1971,7 +1992,7 @@ void launch_bwd(const agpt_attn_s* h, const void* q, const void* k, const void* 
         hipLaunchKernelGGL(fc, dim3(grid), dim3(agpt_deep::kThreads), lds, st, plan_dev(h),
                            static_cast<const Tin*>(q), static_cast<const Tin*>(k), static_cast<const Tin*>(v), lse,
                            h->d_Dl, static_cast<const Tin*>(dO), dk, dv, h->d_E, h->d_F, h->d_Cs, acc_dk, acc_dv,
-                           rope, h->cfg.n_heads, scale);
+                           rope_kv, h->cfg.n_heads, scale);
         pm.mark(2);
         pm.mark(3);
         launch_carry<HD>(h, dk, dv, acc_dk, acc_dv, rope, st);

@@ -60,10 +60,9 @@ constexpr int kThreads = 256;
 constexpr int kChunk = 64;  // keys per streamed chunk: one 16-key block per wave-sized step
 constexpr int kKeyCap = (kMaxDepth - 1 + kTile + kChunk - 1) / kChunk * kChunk;
 // Key blocks per wave of the carry key side with its sums in registers:
-// kRegItersDeep blocks per wave (key slots 0 .. 16 * 4 * kRegItersDeep - 1),
-// the default; or, on request, every key slot of a tile of a plan to depth
-// kRegDepth (prefix_cap + 64 keys in 4 kRegIters blocks of 16), which at
-// the register limit spills inside the key-block loop.
+// every key slot of a tile (prefix_cap + 64 keys in 4 blocks of 16 per turn)
+// in kRegItersDeep blocks per wave for plans to depth 65, in kRegIters for
+// plans to depth kRegDepth; deeper plans keep their first kRegItersDeep.
 constexpr int kRegIters = 3;
 constexpr int kRegDepth = 4 * kRegIters * 16 - kTile;  // 128
 constexpr int kRegItersDeep = 2;
@@ -555,6 +554,10 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(kOnePa
   const int64_t n_units = static_cast<int64_t>(pl.n_tiles) * ngr;
   Claims claims = make_claims(pl, 1, n_units);
   if (threadIdx.x == 0) tb.next[1] = claims.next();
+  // (The one-pass bf16 kernel reads the caller's rope tables: with the table
+  // in LDS it spills 14 registers.)
+  agpt_blk::RopeTab<HD, RopeT> rt(rope, dyn + ring_lds_bytes(HD, sizeof(Tin)));
+  if constexpr (!kOnePass) rt.fill();
   __syncthreads();
   int u = uniform(tb.next[1]);
   for (int par = 0; u < n_units; par ^= 1) {
@@ -716,7 +719,11 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(kOnePa
 #pragma unroll
           for (int j = 0; j < MT; ++j) {
             float v[4] = {dq[j][0], dq[j][1], dq[j][2], dq[j][3]};
-            if (rope.cos_t) agpt_fast::rope_inverse_part<4, HD>(v, rope.cos_t, rope.sin_t, pos, kBlk * j + 4 * g);
+            if constexpr (kOnePass) {
+              if (rope.cos_t) agpt_fast::rope_inverse_part<4, HD>(v, rope.cos_t, rope.sin_t, pos, kBlk * j + 4 * g);
+            } else {
+              if (rt) rt.inverse(v, qdep, kBlk * j + 4 * g);
+            }
             store_vec<4>(dQ + row * D + h * HD + kBlk * j + 4 * g, v);
           }
           if (g == 0) Dl[row * H + h] = dl;
@@ -1165,10 +1172,10 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(sizeof
   }
 }
 
-// The key side's K/V slice cache (bf16, every key slot in registers: NI ==
-// kRegIters): per wave and register block, four 16-byte pieces per lane.
-__host__ __device__ constexpr size_t kv_cache_bytes(int ni, int elem) {
-  return ni == kRegIters && elem == 2 ? static_cast<size_t>(kThreads / 64) * kRegIters * 4 * 64 * 16 : 0;
+// The key side's K/V slice cache (bf16, every key slot in registers: kAll):
+// per wave and register block, four 16-byte pieces per lane.
+__host__ __device__ constexpr size_t kv_cache_bytes(int ni, bool all, int elem) {
+  return all && elem == 2 ? static_cast<size_t>(kThreads / 64) * ni * 4 * 64 * 16 : 0;
 }
 static_assert(rows_lds_bytes(64, 2) % 16 == 0 && RawTabs::kBytes % 16 == 0, "16-byte aligned cache entries");
 // A 16-dim bf16 slice from / to two 16-byte pieces.
@@ -1209,8 +1216,10 @@ __device__ __forceinline__ int opaque_tid() {
 // chains). With NI > 0 the wave that owns a key block keeps the block's
 // sums in registers, as the accumulators of its matrix products, from one
 // tile to the next: a key that stays in its slot never leaves them. NI ==
-// kRegItersDeep covers the first 16 * 4 NI slots of a tile; NI == kRegIters
-// (plans to depth kRegDepth) covers every key slot.
+// kRegItersDeep covers the first 16 * 4 NI slots of a tile; with kAll the NI
+// blocks per wave cover every key slot (kRegIters for plans to depth
+// kRegDepth; kRegItersDeep for plans to depth 65, whose fewer sums leave the
+// fp32 kernel without spills).
 // The other sums go through this workgroup's carry rows Cs
 // [parity][depth][dK, dV][HD] (global memory, read and written only by this
 // workgroup; a tile reads the rows of its parity and writes the next
@@ -1226,7 +1235,7 @@ __device__ __forceinline__ int opaque_tid() {
 // chunks, in chunk order).
 // E, F: [n_chunks][P][2][D].
 // ---------------------------------------------------------------------------
-template <int HD, typename Tin, int NI, typename PlanT, typename RopeT>
+template <int HD, typename Tin, int NI, bool kAll, typename PlanT, typename RopeT>
 __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(NI > 0 ? 2 : 3))) void bwd_kv_carry_kernel(
     PlanT pl, const Tin* __restrict__ Q, const Tin* __restrict__ K, const Tin* __restrict__ V,
     const float* __restrict__ lse, const float* __restrict__ Dl, const Tin* __restrict__ dO,
@@ -1246,7 +1255,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(NI > 0
   Tin* Qs = reinterpret_cast<Tin*>(dyn);
   Tin* Gs = Qs + kTile * WS;
   const RawTabs raw{reinterpret_cast<int32_t*>(dyn + rows_lds_bytes(HD, sizeof(Tin)))};
-  constexpr bool kCache = kv_cache_bytes(NI, sizeof(Tin)) > 0;
+  constexpr bool kCache = kv_cache_bytes(NI, kAll, sizeof(Tin)) > 0;
   u4* const kvc = reinterpret_cast<u4*>(dyn + rows_lds_bytes(HD, sizeof(Tin)) + RawTabs::kBytes) +
                   (kCache ? (threadIdx.x >> 6) * NI * 4 * 64 : 0);
   const int lane = threadIdx.x & 63;
@@ -1262,6 +1271,9 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(NI > 0
   const int64_t n_units = static_cast<int64_t>(pl.n_chunks) * H;
   int* ctr = pl.sched + 2;
   if (threadIdx.x == 0) tb.next[1] = atomicAdd(ctr, 1);
+  agpt_blk::RopeTab<HD, RopeT> rt(
+      rope, dyn + rows_lds_bytes(HD, sizeof(Tin)) + RawTabs::kBytes + kv_cache_bytes(NI, kAll, sizeof(Tin)));
+  rt.fill();
   __syncthreads();
   int u = uniform(tb.next[1]);
   for (int par = 0; u < n_units; par ^= 1) {
@@ -1473,7 +1485,6 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(NI > 0
         };
         // Final dK/dV of row a at depth dep: + seeds, inverse RoPE of dK.
         auto finish = [&](int64_t a, int dep) {
-          const int pos = rope.cos_t ? rope_pos(dep, rope.seq_len) : 0;
 #pragma unroll
           for (int j = 0; j < MT; ++j) {
             const int d0 = kBlk * j + 4 * g;
@@ -1489,7 +1500,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(NI > 0
 #pragma unroll
               for (int x = 0; x < 4; ++x) gv[j][x] += y[x];
             }
-            if (rope.cos_t) agpt_fast::rope_inverse_part<4, HD>(gk[j], rope.cos_t, rope.sin_t, pos, d0);
+            if (rt) rt.inverse(gk[j], dep, d0);
             store_vec<4>(dK + a * D + h * HD + d0, gk[j]);
             store_vec<4>(dV + a * D + h * HD + d0, gv[j]);
           }
@@ -1551,7 +1562,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(NI > 0
         if constexpr (kCache) fetch_c(wave, 0, nkf, nvf, nmiss);
         else fetch(wave, nkf, nvf);
       }
-      if constexpr (NI == kRegIters) {  // every key block of the tile in registers
+      if constexpr (kAll) {  // every key block of the tile in registers
 #pragma unroll
         for (int i = 0; i < NI; ++i)
           if (wave + 4 * i < nkb) key_block(wave + 4 * i, ck[i], cv[i], true, i);
