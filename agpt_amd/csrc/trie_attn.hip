@@ -417,7 +417,11 @@ __global__ __launch_bounds__(256) void trie_bwd_kernel(
 // Reduction level 1: chunk c (kChunkTiles consecutive tiles) sums the prefix
 // partials of slot k over its tiles, for the slots every tile of the chunk
 // has (k < min A). Such a sum is used only when the whole chunk lies inside
-// one key's span, where slot k names the same key in every tile.
+// one key's span, where slot k names the same key in every tile. A thread
+// takes 4 columns of one slot; blockIdx.y splits a chunk's columns, so that
+// plans of few chunks fill the chip too (16 chunks of 8 x 64 at depth 128, one
+// workgroup each: 1.50 ms), with eight tiles' loads in flight: 891K rows of
+// 8 x 16 73 -> 15 us, 925K rows to depth 64 197 -> 17 us.
 // ---------------------------------------------------------------------------
 __global__ __launch_bounds__(256) void trie_bwd_chunk_kernel(PlanDev pl, const float* __restrict__ Pk,
                                                              const float* __restrict__ Pv,
@@ -425,27 +429,36 @@ __global__ __launch_bounds__(256) void trie_bwd_chunk_kernel(PlanDev pl, const f
                                                              float* __restrict__ Cv, int D) {
   const int c = blockIdx.x;
   const int u0 = c * kChunkTiles;
-  const int u1 = min(pl.n_tiles, u0 + kChunkTiles);
+  const int nu = min(pl.n_tiles - u0, kChunkTiles);
+  __shared__ int offs[kChunkTiles + 1];
   __shared__ int min_a;
+  if (threadIdx.x <= nu) offs[threadIdx.x] = pl.pref_off[u0 + threadIdx.x];
+  __syncthreads();
   if (threadIdx.x == 0) {
     int m = kMaxDepth;
-    for (int u = u0; u < u1; ++u) m = min(m, pl.pref_off[u + 1] - pl.pref_off[u]);
+    for (int u = 0; u < nu; ++u) m = min(m, offs[u + 1] - offs[u]);
     min_a = m;
   }
   __syncthreads();
-  const int total = min_a * D;
-  for (int idx = threadIdx.x; idx < total; idx += blockDim.x) {
-    const int k = idx / D;
-    const int col = idx - k * D;
-    float sk = 0.0f, sv = 0.0f;
-    for (int u = u0; u < u1; ++u) {
-      const int64_t row = static_cast<int64_t>(pl.pref_off[u]) + k;
-      sk += Pk[row * D + col];
-      sv += Pv[row * D + col];
+  const int Q = D / 4;
+  const int total = 2 * min_a * Q;  // (slot, K or V, 4 columns)
+  for (int idx = blockIdx.y * blockDim.x + threadIdx.x; idx < total; idx += gridDim.y * blockDim.x) {
+    const int k = idx / (2 * Q);
+    const int tv = (idx - k * 2 * Q) / Q;
+    const int col = (idx % Q) * 4;
+    const float* src = (tv ? Pv : Pk) + static_cast<int64_t>(k) * D + col;
+    float v[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+    for (int u = 0; u < nu; u += 8) {
+      float y[8][4];
+#pragma unroll
+      for (int x = 0; x < 8; ++x) load_vec<4>(src + static_cast<int64_t>(offs[min(u + x, nu - 1)]) * D, y[x]);
+#pragma unroll
+      for (int x = 0; x < 8; ++x)
+        if (u + x < nu)
+#pragma unroll
+          for (int e = 0; e < 4; ++e) v[e] += y[x][e];
     }
-    const int64_t o = (static_cast<int64_t>(c) * pl.max_depth + k) * D + col;
-    Ck[o] = sk;
-    Cv[o] = sv;
+    store_vec<4>((tv ? Cv : Ck) + (static_cast<int64_t>(c) * pl.max_depth + k) * D + col, v);
   }
 }
 
@@ -454,6 +467,10 @@ __global__ __launch_bounds__(256) void trie_bwd_chunk_kernel(PlanDev pl, const f
 // the prefix path of tile t+1). dK_a = own-tile partial (already in dK) +
 // Σ over tiles u in (t, tile(end_a - 1)] of slot depth(a)-1, in tile order,
 // using chunk sums for whole chunks. Then seeds, inverse RoPE, final write.
+// Bound by the rows' round trip (dK, dV read and written, the partials read:
+// 0.7 GB in 179 us for 891K rows of 8 x 16); a wave fetches the rows and
+// subtree ends of all its keys at once (lane i: its i-th key) and takes them
+// out by lane (192 -> 179 us).
 // ---------------------------------------------------------------------------
 // VW consecutive columns per lane: one walk over the tiles covers 64 * VW
 // columns (D = 512 in one walk with VW = 8, 16-byte loads).
@@ -504,10 +521,15 @@ __global__ __launch_bounds__(256) void trie_bwd_reduce_kernel(
   const int wave = threadIdx.x >> 6;
   const int lane = threadIdx.x & 63;
   const int nwaves = blockDim.x >> 6;
-  for (int k = An - 1 - wave; k >= 0; k -= nwaves) {
-    const int64_t a = pl.prefix[noff + k];
+  // At most kMaxDepth / nwaves = 64 keys per wave.
+  static_assert(kMaxDepth <= 64 * 4, "a lane per key of the wave");
+  const int kl = An - 1 - wave - nwaves * lane;
+  const int key_row = kl >= 0 ? pl.prefix[noff + kl] : -1;
+  const int key_end = kl >= 0 ? pl.pref_end[noff + kl] : 0;
+  for (int n = 0, k = An - 1 - wave; k >= 0; ++n, k -= nwaves) {
+    const int64_t a = __builtin_amdgcn_readlane(key_row, n);
     if (a < s) break;  // deeper-first scan: everything above is outside tile t
-    const int u_last = static_cast<int>((pl.end[a] - 1) / pl.tile);
+    const int u_last = (__builtin_amdgcn_readlane(key_end, n) - 1) / pl.tile;
     const int pos = rope.cos_t ? rope_pos(k + 1, rope.seq_len) : 0;
     for (int col0 = lane * VW; col0 < D; col0 += 64 * VW) {
       float sk[VW], sv[VW];
@@ -520,7 +542,7 @@ __global__ __launch_bounds__(256) void trie_bwd_reduce_kernel(
       while (u <= u_last) {
         const float* srck[kR];
         const float* srcv[kR];
-        int n = 0;
+        int n = 0;  // parts of this round
         for (; n < kR && u <= u_last; ++n) {
           const int c = u / kChunkTiles;
           if (u == c * kChunkTiles && u + kChunkTiles - 1 <= u_last) {
@@ -529,7 +551,7 @@ __global__ __launch_bounds__(256) void trie_bwd_reduce_kernel(
             srcv[n] = Cv + o;
             u += kChunkTiles;
           } else {
-            const int64_t o = (static_cast<int64_t>(pl.pref_off[u]) + k) * D + col0;
+            const int64_t o = (static_cast<int64_t>(u == t + 1 ? noff : pl.pref_off[u]) + k) * D + col0;
             srck[n] = Pk + o;
             srcv[n] = Pv + o;
             ++u;
@@ -1342,8 +1364,9 @@ int plan_impl(agpt_attn_s* h, const int32_t* ext, int64_t n_ext, int32_t A0,
     // deep key side). Below that, at least 3 tiles while every workgroup (2
     // per CU) still gets a claim: each chunk reads its first tile's prefix
     // from memory and writes E and F rows for the carry kernel. The deep key
-    // side takes 2 at least: chunks of one tile carry nothing and leave
-    // per-tile partials. Without a carry (the split block kernels) long chunks
+    // side takes 2 at least where its per-tile partials (what chunks of one
+    // tile leave) are more than a static plan could hold: below that both
+    // plans keep the partials, and give the same bytes. Without a carry (the split block kernels) long chunks
     // only save prefix reads: 4 at most. Forward + backward, 8 claims per CU
     // and no floor against this rule: 31K rows of 8 x 64 bf16, depth 128, 1.67
     // ms (chunks of 1) -> 0.30 (3); 767K of 4 x 32 1.91 (23) -> 1.69 (11);
@@ -1355,7 +1378,10 @@ int plan_impl(agpt_attn_s* h, const int32_t* ext, int64_t n_ext, int32_t A0,
     const int64_t claims1 = static_cast<int64_t>(n_tiles) *  // claims of one tile
                             (h->deep_carry ? h->cfg.n_heads : std::max(1, h->cfg.n_heads / std::max(1, h->hg)));
     const int64_t cap = h->deep_carry ? 96 : h->carry ? 24 : 4;
-    const int64_t lo = std::max<int64_t>(h->deep_carry ? 2 : 1, std::min<int64_t>(3, claims1 / (2 * cus)));
+    const bool big_partials = static_cast<size_t>(pref_off[n_tiles]) * h->cfg.n_heads * h->cfg.head_dim * 8 > kScratchBytes;
+    const int64_t lo = h->deep_carry && !big_partials
+                           ? 1
+                           : std::max<int64_t>(h->deep_carry ? 2 : 1, std::min<int64_t>(3, claims1 / (2 * cus)));
     const int per_cu = h->cfg.dtype == AGPT_DTYPE_BF16 || (h->fused && h->cfg.head_dim == 32) ? 16 : 8;
     const int dflt = static_cast<int>(std::min(cap, std::max(lo, claims1 / (per_cu * cus))));
     h->chunk_tiles = std::max(1, env_int("AGPT_ATTN_CHUNK", dflt));
@@ -1368,6 +1394,14 @@ int plan_impl(agpt_attn_s* h, const int32_t* ext, int64_t n_ext, int32_t A0,
                                 : 0;
   }
   auto fl = [&](float** p, size_t bytes) { return ar.get(reinterpret_cast<void**>(p), bytes); };
+  // A static plan that the carry's partials would push past the scratch keeps
+  // per-tile partials, which take less for short chunks.
+  if (ar.base && h->carry && h->cfg.head_dim == 32 &&
+      ar.used + static_cast<size_t>(h->n_chunks_sched) * agpt_blk::prefix_cap(maxd) * 4 * D * sizeof(float) +
+              static_cast<size_t>(n) * h->cfg.n_heads * sizeof(float) + 1024 > kScratchBytes) {
+    h->carry = h->rope_lds = false;
+    h->fb_lds = agpt_blk::fused_lds_bytes(h->max_depth, h->fhg, h->cfg.head_dim, false);
+  }
   if (h->carry || h->deep_carry) {
     const size_t ebytes = static_cast<size_t>(h->n_chunks_sched) * agpt_blk::prefix_cap(maxd) * 2 * D * sizeof(float);
     if ((rc = fl(&h->d_E, ebytes)) != AGPT_OK || (rc = fl(&h->d_F, ebytes)) != AGPT_OK) return rc;
@@ -2059,7 +2093,8 @@ void launch_bwd(const agpt_attn_s* h, const void* q, const void* k, const void* 
   }
   pm.mark(2);
   if (h->n_tiles > 1) {
-    hipLaunchKernelGGL(trie_bwd_chunk_kernel, dim3(h->n_chunks), dim3(256), 0, st, plan_dev(h), h->d_Pk,
+    const int split = std::max(1, std::min((h->max_depth * D / 2 + 255) / 256, (2048 + h->n_chunks - 1) / h->n_chunks));
+    hipLaunchKernelGGL(trie_bwd_chunk_kernel, dim3(h->n_chunks, split), dim3(256), 0, st, plan_dev(h), h->d_Pk,
                        h->d_Pv, h->d_Ck, h->d_Cv, D);
     pm.mark(3);
     auto reduce = [&](auto vw) {

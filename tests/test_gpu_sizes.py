@@ -84,3 +84,38 @@ def test_default_chunk_lengths(gpu, H, hd, dtype, rows):
     tr = small_trie(n_tokens=26000, order=4, vocab=30, depth=12, seed=9)
     assert tr.n_nodes >= rows
     _check(tr.parent[:rows], H, hd, seed=rows, dtype=dtype, rope=True)
+
+
+@pytest.mark.parametrize("H,hd,dtype,rows", [(3, 16, "f32", 33 * 64 + 5), (1, 16, "f32", 32 * 64), (2, 64, "f32", 70 * 64 + 1),
+                                             (4, 64, "bf16", 65 * 64)])
+def test_partial_sums_over_chunks(gpu, monkeypatch, H, hd, dtype, rows):
+    """Without the carry: chunk sums of the per-tile partials over whole and
+    short 32-tile chunks, one root over all of them."""
+    monkeypatch.setenv("AGPT_ATTN_CARRY", "0")
+    par = _tree(rows - 1, 20, seed=rows)
+    par = np.concatenate([[-1], par + 1]).astype(np.int32)
+    _check(par, H, hd, seed=rows, dtype=dtype, rope=dtype == "f32", acc=dtype == "f32")
+
+
+def test_static_plan_past_the_carry(gpu):
+    """A batch at head_dim 32 whose carry partials would not fit the static
+    scratch, but whose per-tile partials do, is still planned there. Its dK/dV
+    sums are grouped by tile instead of by chunk: equal to the allocated
+    plan's within the sums' fp32 rounding (root keys sum ~1e5 terms)."""
+    import torch
+
+    from agpt_amd import trie
+    from agpt_amd.attention import TrieAttention
+    par = trie.build_radix_trie(trie.markov_corpus(6800, 3, 65, 1.1, 4), 32).parent
+    q, k, v, g = (torch.from_numpy(x).cuda() for x in tensors(par.shape[0], 128, 3))
+    outs = []
+    for static in (True, False):
+        att = TrieAttention(4, 32, max_depth=32)
+        (att.plan_static if static else att.plan)(par)
+        assert ("path-carry" in att.describe()) != static
+        o, lse = att.forward(q, k, v)
+        outs.append((o, lse) + tuple(att.backward(q, k, v, o, lse, g)))
+        torch.cuda.synchronize()
+        att.close()
+    for name, a, b in zip(("O", "lse", "dQ", "dK", "dV"), *outs):
+        assert (a - b).norm() <= 2e-6 * b.norm(), name
