@@ -375,8 +375,20 @@ constexpr int kLqMaxDelta = 1024;  // queries per node in the backward's per-wav
 
 __device__ __forceinline__ int lq_uniform(int v) { return __builtin_amdgcn_readfirstlane(v); }
 
+// Orders a wave's LDS writes before its other lanes' reads, and those before
+// the next writes. The hardware keeps a wave's LDS operations in order; this
+// holds the compiler to it, at no instruction.
+__device__ __forceinline__ void lq_lds_order() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront", "local");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront", "local");
+}
+
 // Element idx from a wave-uniform base as a 32-bit byte offset (a scalar base
-// and one register per address; a node's rows and weights span < 4 GiB).
+// and one register per address). A block of 16 rows spans < 4 GiB; a whole
+// node's weights may not (8,200 queries of 16 heads: 4.3 GB), nor its packed
+// rows, so in the forward their base moves with the block. Its queries do:
+// L rows of them come with at least L * L * H weights.
 __device__ __forceinline__ const float* lq_at(const float* base, uint32_t idx) {
   return reinterpret_cast<const float*>(reinterpret_cast<const char*>(base) + idx * 4u);
 }
@@ -450,7 +462,7 @@ constexpr int kLqCache = 4;
 // normalized weights (visible entries only) and adds O^T += V^T P^T.
 // Bound by the latency of each node's chain of loads, hence by the waves in
 // flight: the loops stay rolled and the addresses are a scalar base with a
-// 32-bit offset, 76 VGPRs for 138 (8 x 16, 1.76M queries: 2.08 -> 1.76 ms).
+// 32-bit offset, 80 VGPRs for 138 (8 x 16, 1.76M queries: 2.08 -> 1.76 ms).
 template <int HD>
 __global__ __launch_bounds__(256) void varlen_Lq_fwd_kernel(
     const float* __restrict__ q, const float* __restrict__ k, const float* __restrict__ v,
@@ -499,7 +511,7 @@ __global__ __launch_bounds__(256) void varlen_Lq_fwd_kernel(
       for (int x = 0; x < kLqCache; ++x) sc[x] = f4{0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll 1
       for (int b = 0; b < pend; b += 16) {
-        const f4 sv0 = lq_rows_dot<HD>(lq_at(kh, min(b + c, len - 1) * RS), qy, g);
+        const f4 sv0 = lq_rows_dot<HD>(lq_at(kh + static_cast<int64_t>(b) * RS, min(c, len - 1 - b) * RS), qy, g);
 #pragma unroll
         for (int x = 0; x < kLqCache; ++x)
           if (b == 16 * x) sc[x] = sv0;
@@ -521,7 +533,7 @@ __global__ __launch_bounds__(256) void varlen_Lq_fwd_kernel(
       f4 o[MT];
 #pragma unroll
       for (int t = 0; t < MT; ++t) o[t] = f4{0.0f, 0.0f, 0.0f, 0.0f};
-      float* wrow = lq_at(wh, static_cast<uint32_t>(qok ? jq : 0) * WS);
+      float* wrow = lq_at(wh + static_cast<int64_t>(i) * WS, static_cast<uint32_t>(qok ? c : 0) * WS);
 #pragma unroll 1
       for (int b = 0; b < pend; b += 16) {
         // V^T operand first: lane (g, c) supplies V[row b + 4g + j][dim 16t + c]
@@ -529,12 +541,14 @@ __global__ __launch_bounds__(256) void varlen_Lq_fwd_kernel(
 #pragma unroll
         for (int j = 0; j < 4; ++j)
 #pragma unroll
-          for (int t = 0; t < MT; ++t) vt[t][j] = *lq_at(vh, min(b + 4 * g + j, len - 1) * RS + 16 * t + c);
+          for (int t = 0; t < MT; ++t)
+            vt[t][j] = *lq_at(vh + static_cast<int64_t>(b) * RS, min(4 * g + j, len - 1 - b) * RS + 16 * t + c);
         f4 sv = sc[0];
 #pragma unroll
         for (int x = 1; x < kLqCache; ++x)
           if (b == 16 * x) sv = sc[x];
-        if (b >= 16 * kLqCache) sv = lq_rows_dot<HD>(lq_at(kh, min(b + c, len - 1) * RS), qy, g);
+        if (b >= 16 * kLqCache)
+          sv = lq_rows_dot<HD>(lq_at(kh + static_cast<int64_t>(b) * RS, min(c, len - 1 - b) * RS), qy, g);
         float pw[4];
         const int vis = qok ? min(len, shift + jq + 1) : 0;  // this query's visible rows
 #pragma unroll
@@ -554,7 +568,8 @@ __global__ __launch_bounds__(256) void varlen_Lq_fwd_kernel(
       // O^T[dim 16t + 4g + r][query c]
       if (qok)
 #pragma unroll
-        for (int t = 0; t < MT; ++t) *reinterpret_cast<f4*>(lq_at(oh, jq * RS + 16 * t + 4 * g)) = o[t];
+        for (int t = 0; t < MT; ++t)
+          *reinterpret_cast<f4*>(lq_at(oh, jq * RS + 16 * t + 4 * g)) = o[t];
     }
   }
 }
@@ -830,12 +845,14 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(HD * NB == 
         for (int t = 0; t < MT; ++t)
 #pragma unroll
           for (int j = 0; j < 4; ++j) dqa[t] = lq_mfma(kt[t][j], ds[j], dqa[t]);
+        lq_lds_order();
         float wv[4], dsv[4];
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
           wv[j] = pt[(4 * g + j) * TS + c];
           dsv[j] = st[(4 * g + j) * TS + c];
         }
+        lq_lds_order();
 #pragma unroll
         for (int j = 0; j < 4; ++j)
 #pragma unroll

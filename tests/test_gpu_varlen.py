@@ -184,3 +184,34 @@ def test_varlen_L_queries_row_limits(gpu, H, hd, longest):
                             dk=S.ravel(), dv=S.ravel())
     for name, got, ref in zip(("dQ", "dK", "dV"), (dq, dk, dv), want):
         assert_close(got.cpu().numpy(), ref, what=name)
+
+
+def test_varlen_L_queries_node_past_4gib(gpu):
+    """A node whose weights alone pass 4 GiB (8,200 queries of 16 heads):
+    output and weights of its first and last queries against float64 softmax
+    attention, at the fp32 bar."""
+    import torch
+
+    from agpt_amd import attention as A
+    H, hd, n = 16, 16, 8200
+    assert n * H * n * 4 > 1 << 32
+    D, scale = H * hd, scale_of(hd)
+    g = torch.Generator(device="cuda")
+    g.manual_seed(1)
+    Q, K, V = (torch.randn(n, D, generator=g, device="cuda") for _ in range(3))
+    q2n = torch.zeros(n, dtype=torch.int32, device="cuda")
+    qoff, off, ln = (torch.tensor(x, dtype=torch.int32, device="cuda") for x in ([0, n], [0], [n]))
+    out, w = torch.zeros(n * D, device="cuda"), torch.zeros(n * H * n, device="cuda")
+    A.batched_varlen_attention_L_queries(Q, K, V, q2n, qoff, off, ln, out, w, n, H, hd, n, scale)
+    k64, v64 = (x.view(n, H, hd).double().cpu().numpy() for x in (K, V))
+    for rows in (slice(0, 20), slice(n - 20, n)):
+        wr = w.view(n, H, n)[rows].cpu().numpy()
+        o = out.view(n, H, hd)[rows].cpu().numpy()
+        q64 = Q.view(n, H, hd)[rows].double().cpu().numpy()
+        for j, row in enumerate(range(n)[rows]):
+            s = np.einsum("hd,phd->hp", q64[j], k64[: row + 1]) * scale
+            p = np.exp(s - s.max(1, keepdims=True))
+            p /= p.sum(1, keepdims=True)
+            assert_close(wr[j, :, : row + 1], p, what=f"W of query {row}")
+            assert not wr[j, :, row + 1:].any()
+            assert_close(o[j], np.einsum("hp,phd->hd", p, v64[: row + 1]), what=f"O of query {row}")
