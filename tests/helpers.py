@@ -14,6 +14,13 @@ RTOL_F32, ATOL_F32 = 1e-4, 1e-5
 RTOL_BF16, ATOL_BF16 = 2e-2, 2e-3
 
 
+def _outside(got, want, bound):
+    """Elements with |got - want| > bound. A NaN or an infinity that only one
+    side has is outside every bound; the same one on both sides is inside."""
+    same = (got == want) | (np.isnan(got) & np.isnan(want))
+    return ~same & ~((np.abs(got - want) <= bound) & np.isfinite(want))
+
+
 def assert_close(got, want, rtol=RTOL_F32, atol=ATOL_F32, what="", row_scale=None):
     """|got - want| <= atol + rtol * |want| elementwise.
 
@@ -31,7 +38,7 @@ def assert_close(got, want, rtol=RTOL_F32, atol=ATOL_F32, what="", row_scale=Non
         mag = np.broadcast_to(m, mag.shape[:1] + (mag.size // mag.shape[0] // row_scale, row_scale)
                               ).reshape(mag.shape)
     bound = atol + rtol * mag
-    bad = err > bound
+    bad = _outside(got, want, bound)
     if bad.any():
         i = np.unravel_index(np.argmax(err - bound), err.shape)
         raise AssertionError(
@@ -170,7 +177,7 @@ def assert_close_or_f64(got, want, f64_rows, rtol=RTOL_F32, atol=ATOL_F32, what=
     bar is held against the true value."""
     got = np.asarray(got, dtype=np.float64)
     want = np.asarray(want, dtype=np.float64)
-    bad = (np.abs(got - want) > atol + rtol * np.abs(want)).any(1)
+    bad = _outside(got, want, atol + rtol * np.abs(want)).any(1)
     rows = np.flatnonzero(bad)
     assert rows.size <= 64, f"{what}: {rows.size} rows outside the bar against the oracle"
     if rows.size:
@@ -359,7 +366,7 @@ def assert_close_terms(got, want, terms_rows, rtol=RTOL_BF16, atol=ATOL_BF16, wh
     got = np.asarray(got, dtype=np.float64)
     want = np.asarray(want, dtype=np.float64)
     err = np.abs(got - want)
-    bad = err > atol + rtol * np.abs(want)
+    bad = _outside(got, want, atol + rtol * np.abs(want))
     n_bad = int(bad.sum())
     print(f"{what}: {bad.size - n_bad} of {bad.size} elements within {rtol}|ref| + {atol} "
           f"({n_bad} exceptions)", flush=True)

@@ -189,7 +189,7 @@ def test_c4_full_size_share(gpu):
     def check(name, got, want, terms):
         got, want, terms = (x.reshape(x.shape[0], -1).double() for x in (got, want, terms))
         err = (got - want).abs()
-        bad = err > ATOL_BF16 + RTOL_BF16 * want.abs()
+        bad = ~(err <= ATOL_BF16 + RTOL_BF16 * want.abs())
         print(f"{name}: {int(bad.sum())} of {bad.numel()} elements outside the elementwise bar", flush=True)
         assert int(bad.sum()) <= 1e-3 * bad.numel(), name
         assert bool((err[bad] <= ATOL_BF16 + RTOL_BF16 * terms[bad]).all()), f"{name}: {float(err.max())}"
@@ -317,7 +317,7 @@ def test_c5_full_size(gpu):
     def check(name, got, want, terms):
         got = got.double()
         err = (got - want).abs()
-        bad = err > ATOL_BF16 + RTOL_BF16 * want.abs()
+        bad = ~(err <= ATOL_BF16 + RTOL_BF16 * want.abs())
         bad_count[name] += int(bad.sum())
         if bool(bad.any()):
             worst[name] = max(worst[name], float((err[bad] / (ATOL_BF16 + RTOL_BF16 * terms[bad])).max()))

@@ -470,3 +470,24 @@ def test_abs_terms_bound_the_oracle():
             assert (np.abs(x) <= t * (1 + 1e-5) + 1e-6).all(), kind
             if pos and kind in ("O", "dV"):
                 np.testing.assert_allclose(t, x, rtol=1e-5, atol=1e-6)
+
+
+def test_comparisons_reject_nan():
+    """A NaN or infinite output is outside every comparison's bar, unless the
+    reference holds the same."""
+    from helpers import assert_close_or_f64, assert_close_terms
+    checks = (assert_close, lambda g, w: assert_close(g, w, row_scale=4),
+              lambda g, w: assert_close_or_f64(g, w, lambda rows: w[rows]),
+              lambda g, w: assert_close_terms(g, w, lambda rows: np.ones((len(rows), 4))))
+    want = np.ones((3, 4), np.float32)
+    for bad in (np.nan, np.inf):
+        got = want.copy()
+        got[1, 2] = bad
+        for check in checks:
+            with pytest.raises(AssertionError):
+                check(got, want)
+            with pytest.raises(AssertionError):
+                check(want, got)
+    assert_close(got, got)
+    got[2, 0] = np.nan
+    assert_close(got, got.copy())
