@@ -835,10 +835,16 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(HD * NB == 
         for (int j = 0; j < 4; ++j)
 #pragma unroll
           for (int t = 0; t < MT; ++t) kt[t][j] = *lq_at(kh, min(16 * b + 4 * g + j, len - 1) * RS + 16 * t + c);
+        // Lanes past the last query hold the first query's dO: their dS is
+        // set, not multiplied, to zero, as a non-finite dO would spread to
+        // rows that its query does not see.
         float ds[4];
 #pragma unroll
-        for (int r = 0; r < 4; ++r)
-          ds[r] = static_cast<float>(static_cast<double>(wp[b][r]) * (static_cast<double>(dw[b][r]) - dot) * dscale);
+        for (int r = 0; r < 4; ++r) {
+          const float x =
+              static_cast<float>(static_cast<double>(wp[b][r]) * (static_cast<double>(dw[b][r]) - dot) * dscale);
+          ds[r] = qok ? x : 0.0f;
+        }
         *reinterpret_cast<f4*>(pt + c * TS + 4 * g) = f4{wp[b][0], wp[b][1], wp[b][2], wp[b][3]};
         *reinterpret_cast<f4*>(st + c * TS + 4 * g) = f4{ds[0], ds[1], ds[2], ds[3]};
 #pragma unroll

@@ -215,3 +215,30 @@ def test_varlen_L_queries_node_past_4gib(gpu):
             assert_close(wr[j, :, : row + 1], p, what=f"W of query {row}")
             assert not wr[j, :, row + 1:].any()
             assert_close(o[j], np.einsum("hp,phd->hd", p, v64[: row + 1]), what=f"O of query {row}")
+
+
+@pytest.mark.parametrize("H,hd,n", [(2, 16, 30), (1, 32, 60), (3, 16, 60), (1, 64, 31)])
+@pytest.mark.parametrize("bad", [np.nan, np.inf])
+def test_varlen_L_queries_nonfinite_stays(gpu, H, hd, n, bad):
+    """A non-finite dO of a node's first query reaches the rows that query
+    sees (its own, row 0) and no block of 16 rows past the one it takes part
+    in: the backward's blocks end in padding lanes that hold the first
+    query's operands (n is no multiple of 16)."""
+    import torch
+
+    from agpt_amd import attention as A
+    D, scale = H * hd, scale_of(hd)
+    Q, K, V, G = tensors(n, D, n + hd)
+    q2n, qoff, off, ln = (np.array(x, np.int32) for x in ([0] * n, [0, n], [0], [n]))
+    _, w = ORC.varlen_L_fwd(Q, K, V, q2n, qoff, off, ln, n, H, hd, n, scale)
+    G[0, 0] = bad
+    want = ORC.varlen_L_bwd(Q, K, V, w, G, q2n, qoff, off, ln, n, H, hd, n, scale, n)
+    cu = lambda x: torch.from_numpy(np.ascontiguousarray(x)).cuda()
+    dq, dk, dv = (torch.zeros(n * D, device="cuda") for _ in range(3))
+    A.batched_varlen_attention_L_queries_backward(cu(Q), cu(K), cu(V), cu(w), cu(G), cu(q2n), cu(qoff), cu(off), cu(ln),
+                                                  dq, dk, dv, n, H, hd, n, scale)
+    for name, got, ref in zip(("dQ", "dK", "dV"), (dq, dk, dv), want):
+        got, ref = got.cpu().numpy().reshape(n, D), np.asarray(ref).reshape(n, D)
+        assert not np.isfinite(got[~np.isfinite(ref)]).any(), f"{name}: a non-finite value vanished"
+        assert np.isfinite(ref[16:]).all()
+        assert_close(got[16:], ref[16:], what=f"{name} past the first block")
