@@ -20,6 +20,7 @@
 #include "common.h"
 #include "../../include/agpt_attn.h"
 
+#include <algorithm>
 #include <cstdarg>
 #include <cstdio>
 #include <string>
@@ -385,10 +386,11 @@ __device__ __forceinline__ void lq_lds_order() {
 }
 
 // Element idx from a wave-uniform base as a 32-bit byte offset (a scalar base
-// and one register per address). A block of 16 rows spans < 4 GiB; a whole
-// node's weights may not (8,200 queries of 16 heads: 4.3 GB), nor its packed
-// rows, so in the forward their base moves with the block. Its queries do:
-// L rows of them come with at least L * L * H weights.
+// and one register per address). In the forward the base moves with the block
+// of 16 queries or rows for the weights (8,200 queries of 16 heads: 4.3 GB) and
+// the packed rows; a node's queries are addressed from its first one (a moving
+// base there costs 6 registers and a wave per SIMD at head_dim 16). Calls in
+// which any of these could span 4 GiB take other kernels (lq_fits).
 __device__ __forceinline__ const float* lq_at(const float* base, uint32_t idx) {
   return reinterpret_cast<const float*>(reinterpret_cast<const char*>(base) + idx * 4u);
 }
@@ -901,6 +903,9 @@ int dispatch(int hd, Fn&& fn) {
   }
 }
 
+// Whether `rows` rows of `floats` floats stay within lq_at's 32-bit byte offsets.
+bool lq_fits(int64_t rows, int64_t floats) { return rows * floats < (int64_t{1} << 30); }
+
 bool bad_dims(int n, int H, int max_len) { return n < 0 || H < 1 || max_len < 1; }
 
 int finish_launch() {
@@ -976,12 +981,17 @@ extern "C" int agpt_varlen_attention_L_queries(const float* q, const float* k, c
     return vset_error(AGPT_ERR_INVALID_ARG, "varlen_L: null pointer");
   const int rc = dispatch(head_dim, [&](auto c) {
     constexpr int HD = decltype(c)::value;
-    if constexpr (HD % 16 == 0) {
+    constexpr int HB = HD % 16 == 0 ? HD : 16;
+    // A node has at most max_kv_len queries. Past lq_at's offsets (from 8,192
+    // heads of 64 and 2,048 queries per node, or 256 MiB of weights per query):
+    // a wave per (query, head group), with 64-bit addresses.
+    const int64_t RS = static_cast<int64_t>(n_heads) * HD, WS = static_cast<int64_t>(n_heads) * max_kv_len;
+    if (HD % 16 == 0 && lq_fits(std::max(16, std::min(T_q, max_kv_len)), RS) && lq_fits(16, WS)) {
       const int64_t waves = (static_cast<int64_t>(T_q) + 63) / 64 * n_heads;  // (block of 64 queries, head)
-      hipLaunchKernelGGL((varlen_Lq_fwd_kernel<HD>), dim3(static_cast<unsigned>((waves + 3) / 4)), dim3(256), 0,
+      hipLaunchKernelGGL((varlen_Lq_fwd_kernel<HB>), dim3(static_cast<unsigned>((waves + 3) / 4)), dim3(256), 0,
                          static_cast<hipStream_t>(stream), q, k, v, query_to_node, query_offsets, kv_offsets,
                          kv_lengths, output, weights_out, T_q, n_heads, max_kv_len, scale);
-    } else {  // head dims 4 and 8: a wave per (query, head group)
+    } else {  // head dims 4 and 8, or wide rows: a wave per (query, head group)
       const int64_t items = static_cast<int64_t>(T_q) * VLanes<HD>(n_heads).slots;
       hipLaunchKernelGGL((varlen_fwd_kernel<HD>), dim3(static_cast<unsigned>((items + 3) / 4)), dim3(256), 0,
                          static_cast<hipStream_t>(stream), q, k, v, kv_offsets, kv_lengths, query_to_node,
@@ -1014,10 +1024,12 @@ extern "C" int agpt_varlen_attention_L_queries_backward(
                            scale);
       };
       // Up to 32 or 64 keys the one-pass kernel (its row blocks' sums fit in
-      // registers; at head_dim 64 up to 32).
+      // registers; at head_dim 64 up to 32), where a node's rows, queries and
+      // weights stay within lq_at's offsets (262,144 heads).
       constexpr int HB = HD % 16 == 0 ? HD : 16;
-      if (max_kv_len <= 32) run(varlen_Lq_bwd_short_kernel<HB, 2>, 0);
-      else if (max_kv_len <= 64 && HB <= 32) run(varlen_Lq_bwd_short_kernel<HB, HB <= 32 ? 4 : 2>, 0);
+      const bool one_pass = lq_fits(max_kv_len, static_cast<int64_t>(n_heads) * std::max(HD, max_kv_len));
+      if (one_pass && max_kv_len <= 32) run(varlen_Lq_bwd_short_kernel<HB, 2>, 0);
+      else if (one_pass && max_kv_len <= 64 && HB <= 32) run(varlen_Lq_bwd_short_kernel<HB, HB <= 32 ? 4 : 2>, 0);
       else run(varlen_Lq_bwd_kernel<HB>, sizeof(double) * 4 * max_kv_len);
     } else {  // head dims 4 and 8, or a δ table past the wave's LDS share: a workgroup per (radix node, head)
       hipLaunchKernelGGL((varlen_L_bwd_kernel<HD>), dim3(T_q, n_heads), dim3(64),

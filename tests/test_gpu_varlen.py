@@ -242,3 +242,66 @@ def test_varlen_L_queries_nonfinite_stays(gpu, H, hd, n, bad):
         assert not np.isfinite(got[~np.isfinite(ref)]).any(), f"{name}: a non-finite value vanished"
         assert np.isfinite(ref[16:]).all()
         assert_close(got[16:], ref[16:], what=f"{name} past the first block")
+
+
+def _f64_heads(Q, K, V, G, heads, hd, n, scale):
+    """float64 (weights, O, dQ, dK, dV) of one node of n queries over its n
+    rows, for the given heads: [len(heads), n, ..]."""
+    q, k, v, g = (x.view(n, -1, hd)[:, heads].double().cpu().numpy().transpose(1, 0, 2) for x in (Q, K, V, G))
+    s = np.einsum("hjd,hpd->hjp", q, k) * scale
+    s = np.where(np.tri(n, dtype=bool), s, -np.inf)
+    w = np.exp(s - s.max(2, keepdims=True))
+    w /= w.sum(2, keepdims=True)
+    dw = np.einsum("hjd,hpd->hjp", g, v)
+    ds = w * (dw - (w * dw).sum(2, keepdims=True)) * scale
+    return (w, np.einsum("hjp,hpd->hjd", w, v), np.einsum("hjp,hpd->hjd", ds, k), np.einsum("hjp,hjd->hpd", ds, q),
+            np.einsum("hjp,hjd->hpd", w, g))
+
+
+@pytest.mark.parametrize("H,hd,n,longest", [(64, 16, 16, 1_200_000), (170_000, 64, 100, 100), (1_100_000, 64, 17, 17)])
+def test_varlen_L_queries_spans_past_4gib(gpu, H, hd, n, longest):
+    """Forward where a block of 16 weight rows spans 4 GiB (a short node in a
+    table of long rows), where one node's queries and packed rows do, and
+    where 17 of them do: all rows of sampled heads against float64."""
+    import torch
+
+    from agpt_amd import attention as A
+    scale = scale_of(hd)
+    g = torch.Generator(device="cuda")
+    g.manual_seed(2)
+    Q, K, V = (torch.randn(n, H * hd, generator=g, device="cuda") for _ in range(3))
+    q2n = torch.zeros(n, dtype=torch.int32, device="cuda")
+    qoff, off, ln = (torch.tensor(x, dtype=torch.int32, device="cuda") for x in ([0, n], [0], [n]))
+    out = torch.zeros(n * H * hd, device="cuda")
+    w = torch.zeros(n * H * longest, device="cuda")
+    A.batched_varlen_attention_L_queries(Q, K, V, q2n, qoff, off, ln, out, w, n, H, hd, longest, scale)
+    heads = [0, 1, H // 2, H - 1]
+    w_ref, o_ref = _f64_heads(Q, K, V, Q, heads, hd, n, scale)[:2]
+    got_w = w.view(n, H, longest)[:, heads, :n].cpu().numpy().transpose(1, 0, 2)
+    assert_close(got_w, w_ref, what="W")
+    assert_close(out.view(n, H, hd)[:, heads].cpu().numpy().transpose(1, 0, 2), o_ref, what="O")
+
+
+def test_varlen_L_queries_backward_weights_past_4gib(gpu):
+    """Backward with rows of 64 keys whose one node's weights pass 4 GiB
+    (272,000 heads): all rows of sampled heads against float64."""
+    import torch
+
+    from agpt_amd import attention as A
+    H, hd, n = 272_000, 16, 64
+    assert (n - 1) * n * H * 4 > 1 << 32
+    scale = scale_of(hd)
+    g = torch.Generator(device="cuda")
+    g.manual_seed(3)
+    Q, K, V, G = (torch.randn(n, H * hd, generator=g, device="cuda") for _ in range(4))
+    q2n = torch.zeros(n, dtype=torch.int32, device="cuda")
+    qoff, off, ln = (torch.tensor(x, dtype=torch.int32, device="cuda") for x in ([0, n], [0], [n]))
+    heads = [0, 1, H // 2, H - 1]
+    w_ref, _, *want = _f64_heads(Q, K, V, G, heads, hd, n, scale)
+    w = torch.zeros(n, H, n, device="cuda")
+    w[:, heads] = torch.from_numpy(w_ref.transpose(1, 0, 2).astype(np.float32)).cuda()
+    dq, dk, dv = (torch.zeros(n * H * hd, device="cuda") for _ in range(3))
+    A.batched_varlen_attention_L_queries_backward(Q, K, V, w.view(-1), G, q2n, qoff, off, ln, dq, dk, dv, n, H, hd, n,
+                                                  scale)
+    for name, got, ref in zip(("dQ", "dK", "dV"), (dq, dk, dv), want):
+        assert_close(got.view(n, H, hd)[:, heads].cpu().numpy().transpose(1, 0, 2), ref, what=name)
