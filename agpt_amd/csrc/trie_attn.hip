@@ -32,6 +32,7 @@
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
+#include <initializer_list>
 #include <mutex>
 #include <string>
 #include <type_traits>
@@ -811,23 +812,33 @@ bool static_plan_current(const agpt_attn_s* h) {
 }
 
 // Device buffers of a plan: hipMalloc, or 256-byte aligned slices of the
-// static scratch. Past the scratch's end it keeps counting (no address is
-// handed out) so the caller can report the bytes the batch needs.
+// static scratch. `used` counts the bytes that the plan takes of the scratch
+// (or would take: both kinds of plan decide by it); past the scratch's end it
+// keeps counting (no address is handed out) so the caller can report the
+// bytes the batch needs.
 struct Arena {
   unsigned char* base = nullptr;  // null: hipMalloc
   size_t used = 0;
   bool overflow = false;
+  static size_t end(size_t used, size_t bytes) {
+    return ((used + 255) & ~static_cast<size_t>(255)) + std::max<size_t>(bytes, 16);
+  }
   int get(void** p, size_t bytes) {
     bytes = std::max<size_t>(bytes, 16);
+    used = end(used, bytes);
     if (!base) {
       HIP_TRY(hipMalloc(p, bytes));
       return AGPT_OK;
     }
-    const size_t off = (used + 255) & ~static_cast<size_t>(255);
-    used = off + bytes;
     if (used > kScratchBytes) overflow = true;
-    *p = overflow ? nullptr : base + off;
+    *p = overflow ? nullptr : base + (used - bytes);
     return AGPT_OK;
+  }
+  // Whether buffers of these sizes would end within the scratch.
+  bool fits(std::initializer_list<size_t> sizes) const {
+    size_t u = used;
+    for (size_t b : sizes) u = end(u, b);
+    return u <= kScratchBytes;
   }
 };
 
@@ -1394,29 +1405,38 @@ int plan_impl(agpt_attn_s* h, const int32_t* ext, int64_t n_ext, int32_t A0,
                                 : 0;
   }
   auto fl = [&](float** p, size_t bytes) { return ar.get(reinterpret_cast<void**>(p), bytes); };
-  // A static plan that the carry's partials would push past the scratch keeps
-  // per-tile partials, which take less for short chunks.
-  if (ar.base && h->carry && h->cfg.head_dim == 32 &&
-      ar.used + static_cast<size_t>(h->n_chunks_sched) * agpt_blk::prefix_cap(maxd) * 4 * D * sizeof(float) +
-              static_cast<size_t>(n) * h->cfg.n_heads * sizeof(float) + 1024 > kScratchBytes) {
-    h->carry = h->rope_lds = false;
-    h->fb_lds = agpt_blk::fused_lds_bytes(h->max_depth, h->fhg, h->cfg.head_dim, false);
+  const size_t pbytes = std::max<size_t>(1, static_cast<size_t>(h->n_prefix_rows) * D) * sizeof(float);
+  const size_t cbytes = std::max<size_t>(1, static_cast<size_t>(h->n_chunks) * maxd * D) * sizeof(float);
+  const size_t dlbytes = static_cast<size_t>(n) * h->cfg.n_heads * sizeof(float);
+  auto ebytes = [&] {
+    return static_cast<size_t>(h->n_chunks_sched) * agpt_blk::prefix_cap(maxd) * 2 * D * sizeof(float);
+  };
+  // At head_dim 32 a batch whose per-tile partials would fit a static plan's
+  // scratch also fits it with the carry: by longer chunks where need be (203K
+  // rows of 4 x 32 to depth 32: 4 tiles for 3), else (nearly no prefixes, or
+  // chunks set by hand) with per-tile partials. Both kinds of plan go by it,
+  // so that they give the same bytes.
+  if (h->carry && h->cfg.head_dim == 32 && ar.fits({pbytes, pbytes, cbytes, cbytes, dlbytes})) {
+    auto fits = [&] { return ar.fits({ebytes(), ebytes(), dlbytes}); };
+    while (!fits() && h->chunk_tiles < 24 && env_int("AGPT_ATTN_CHUNK", 0) == 0)
+      h->n_chunks_sched = std::max<int32_t>(1, n_tiles / ++h->chunk_tiles);
+    if (!fits()) {
+      h->carry = h->rope_lds = false;
+      h->fb_lds = agpt_blk::fused_lds_bytes(h->max_depth, h->fhg, h->cfg.head_dim, false);
+    }
   }
   if (h->carry || h->deep_carry) {
-    const size_t ebytes = static_cast<size_t>(h->n_chunks_sched) * agpt_blk::prefix_cap(maxd) * 2 * D * sizeof(float);
-    if ((rc = fl(&h->d_E, ebytes)) != AGPT_OK || (rc = fl(&h->d_F, ebytes)) != AGPT_OK) return rc;
+    if ((rc = fl(&h->d_E, ebytes())) != AGPT_OK || (rc = fl(&h->d_F, ebytes())) != AGPT_OK) return rc;
     if (h->deep_carry &&
         (rc = fl(&h->d_Cs, static_cast<size_t>(h->cs_slots) * 2 * agpt_blk::prefix_cap(maxd) * 2 *
                                h->cfg.head_dim * sizeof(float))) != AGPT_OK)
       return rc;
   } else if (!h->deep_range) {
-    const size_t pbytes = std::max<size_t>(1, static_cast<size_t>(h->n_prefix_rows) * D) * sizeof(float);
     if ((rc = fl(&h->d_Pk, pbytes)) != AGPT_OK || (rc = fl(&h->d_Pv, pbytes)) != AGPT_OK) return rc;
-    const size_t cbytes = std::max<size_t>(1, static_cast<size_t>(h->n_chunks) * maxd * D) * sizeof(float);
     if ((rc = fl(&h->d_Ck, cbytes)) != AGPT_OK || (rc = fl(&h->d_Cv, cbytes)) != AGPT_OK) return rc;
   }
   if (h->variant == 5 || h->variant == 6)
-    if ((rc = fl(&h->d_Dl, static_cast<size_t>(n) * h->cfg.n_heads * sizeof(float))) != AGPT_OK) return rc;
+    if ((rc = fl(&h->d_Dl, dlbytes)) != AGPT_OK) return rc;
   if (ar.overflow)
     return set_error(AGPT_ERR_INVALID_ARG,
                      "agpt_attn_plan_static: the batch needs %zu bytes of device tables and workspace, more "

@@ -154,9 +154,12 @@ int agpt_attn_plan_range(agpt_attn_handle h, const int32_t* parent, int64_t n_to
  * memory (tight serving loops, harnesses that forbid hipMalloc, code that
  * captures fwd/bwd into a HIP graph: plan before the capture, since the
  * uploads here are synchronous hipMemcpy calls, which a capture does not
- * allow; fwd/bwd of the plan may then be captured). Same contract and results as agpt_attn_plan, but every
- * device table and workspace of the plan is placed in a static array of the
- * library (AGPT_STATIC_SCRATCH_BYTES = 64 MiB per device, held until the
+ * allow; fwd/bwd of the plan may then be captured). Same contract and, to
+ * head_dim 32, the same bytes as agpt_attn_plan (at head_dim 64 a static plan
+ * never carries path sums, so dK/dV of a batch large enough for an allocated
+ * plan to carry them are grouped differently and equal to fp32 rounding), but
+ * every device table and workspace of the plan is placed in a static array of
+ * the library (AGPT_STATIC_SCRATCH_BYTES = 64 MiB per device, held until the
  * process ends) instead of being allocated: the call makes no hipMalloc or
  * hipFree (its only device calls are hipMemcpy uploads of the tables and,
  * once per device, hipGetSymbolAddress). A batch needing more returns

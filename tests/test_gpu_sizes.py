@@ -184,7 +184,8 @@ def test_nan_stays_near_with_carry(gpu, monkeypatch, H, hd, dtype, where):
     test_nan_surfaces(gpu, dtype, H, hd, where)
 
 
-@pytest.mark.parametrize("H,hd,dtype,rows", [(3, 16, "f32", 33 * 64 + 5), (1, 16, "f32", 32 * 64), (2, 64, "f32", 70 * 64 + 1),
+@pytest.mark.parametrize("H,hd,dtype,rows", [(3, 16, "f32", 33 * 64 + 5), (1, 16, "f32", 32 * 64), (2, 32, "f32", 70 * 64 + 1),
+                                             (2, 64, "f32", 70 * 64 + 1),
                                              (4, 64, "bf16", 65 * 64)])
 def test_partial_sums_over_chunks(gpu, monkeypatch, H, hd, dtype, rows):
     """Without the carry: chunk sums of the per-tile partials over whole and
@@ -195,25 +196,31 @@ def test_partial_sums_over_chunks(gpu, monkeypatch, H, hd, dtype, rows):
     _check(par, H, hd, seed=rows, dtype=dtype, rope=dtype == "f32", acc=dtype == "f32")
 
 
-def test_static_plan_past_the_carry(gpu):
+@pytest.mark.parametrize("chunk", [0, 3])
+def test_static_plan_past_the_carry(gpu, monkeypatch, chunk):
     """A batch at head_dim 32 whose carry partials would not fit the static
-    scratch, but whose per-tile partials do, is still planned there. Its dK/dV
-    sums are grouped by tile instead of by chunk: equal to the allocated
-    plan's within the sums' fp32 rounding (root keys sum ~1e5 terms)."""
+    scratch at the default chunk length (3 tiles), but whose per-tile partials
+    do: planned there with longer chunks, or, with the length set by hand, with
+    per-tile partials. The allocated plan does the same: equal bytes."""
     import torch
 
     from agpt_amd import trie
     from agpt_amd.attention import TrieAttention
+    if chunk:
+        monkeypatch.setenv("AGPT_ATTN_CHUNK", str(chunk))
     par = trie.build_radix_trie(trie.markov_corpus(6800, 3, 65, 1.1, 4), 32).parent
-    q, k, v, g = (torch.from_numpy(x).cuda() for x in tensors(par.shape[0], 128, 3))
+    rows = par.shape[0]
+    acc = [torch.from_numpy(x).cuda() for x in tensors(rows, 128, 4, n=2)]
+    rope = [torch.from_numpy(x).cuda() for x in ORC.rope_table(64, 32)]
+    q, k, v, g = (torch.from_numpy(x).cuda() for x in tensors(rows, 128, 3))
     outs = []
     for static in (True, False):
         att = TrieAttention(4, 32, max_depth=32)
         (att.plan_static if static else att.plan)(par)
-        assert ("path-carry" in att.describe()) != static
+        assert ("path-carry" in att.describe()) == (chunk == 0)
         o, lse = att.forward(q, k, v)
-        outs.append((o, lse) + tuple(att.backward(q, k, v, o, lse, g)))
+        outs.append((o, lse) + tuple(att.backward(q, k, v, o, lse, g, acc_dk=acc[0], acc_dv=acc[1], rope=rope)))
         torch.cuda.synchronize()
         att.close()
     for name, a, b in zip(("O", "lse", "dQ", "dK", "dV"), *outs):
-        assert (a - b).norm() <= 2e-6 * b.norm(), name
+        assert torch.equal(a, b), name

@@ -36,7 +36,7 @@ def _fwd_bwd(att, inp, out, rope):
     att.backward(Q, K, V, o, lse, G, acc_dk=acc[0], acc_dv=acc[1], rope=rope, out=(dq, dk, dv))
 
 
-@pytest.mark.parametrize("H,hd", [(8, 16), (2, 64)])
+@pytest.mark.parametrize("H,hd", [(8, 16), (4, 32), (2, 64)])
 def test_plan_static_matches_plan(gpu, H, hd):
     import torch
 
