@@ -1650,9 +1650,12 @@ __global__ __launch_bounds__(kThreads, (kBwdWaves<HD, HG, kCarry>)) void bwd_ker
 // are bound by the latency of their loads: the workgroup's 8 waves fetch 32
 // chunks at a time through LDS, the next 32 in flight while one wave adds
 // them in chunk order. The others, most of the keys, take one thread per 4
-// columns; blockIdx.y spreads them where there are few chunks. 744K rows of
-// 8 x 64 in 258 chunks: 187 -> 57 us (E and F are 270 MB: 55 us at the copy
-// rate).
+// columns; blockIdx.y spreads them where there are few chunks. 31.5M rows of
+// 8 x 16 (20.5K chunks) 263 us; with the fetched chunks through scratch (an
+// array of HIP's float4 does not become registers) 390, with one thread per 4
+// columns of every sum 310. 744K rows of 8 x 64 (528 chunks) 99 us, the time
+// that its E and F (550 MB) take to read; 29K rows of a two-symbol corpus 28,
+// through scratch 41.
 // ---------------------------------------------------------------------------
 constexpr int kCarryThreads = 512;
 constexpr int kLongSum = 16;
@@ -1683,14 +1686,14 @@ __global__ __launch_bounds__(kCarryThreads) void bwd_carry_kernel(
     float* __restrict__ dV, const float* __restrict__ acc_dk, const float* __restrict__ acc_dv, RopeT rope, int H) {
   constexpr int kFetch = 4;                            // chunks a wave fetches per round of a long sum
   constexpr int kRound = kFetch * kCarryThreads / 64;  // chunks per round
-  __shared__ float4 part[kRound][64];
+  __shared__ f4 part[kRound][64];
   const int C = blockIdx.x;
   const int K = pl.chunk_tiles;
   const int64_t rows_per_chunk = static_cast<int64_t>(K) * kTile;
   const int64_t sC = C * rows_per_chunk;
   const int t1 = (C + 1) * K;
   const int off = pl.pref_off[t1];
-  const int A = pl.pref_off[t1 + 1] - off;  // < kMaxDepth <= kCarryThreads
+  const int A = pl.pref_off[t1 + 1] - off;
   const int P = prefix_cap(pl.max_depth);
   const int D = H * HD;
   const int Q = D / 2;  // 4-float jobs of a row: dK then dV
@@ -1699,11 +1702,15 @@ __global__ __launch_bounds__(kCarryThreads) void bwd_carry_kernel(
     return static_cast<int>(min(static_cast<int64_t>(pl.n_chunks), (ea + rows_per_chunk - 1) / rows_per_chunk));
   };
   const int tid = threadIdx.x;
-  const bool entry = tid < A;
-  const int64_t ea = entry ? pl.pref_end[off + tid] : 0;
-  const bool own = entry && pl.prefix[off + tid] >= sC;  // else summed by its own chunk's job
-  const int d0 = A - __syncthreads_count(own);
-  const int nlong = __syncthreads_count(own && c_end(ea) - (C + 1) > kLongSum);
+  const int lane = tid & 63;
+  // Entries below d0 are summed by their own chunk's jobs. Each wave counts
+  // for itself, 64 entries a turn.
+  int d0 = 0, nlong = 0;
+  for (int d = lane; d - lane < A; d += 64) {
+    const bool own = d < A && pl.prefix[off + d] >= sC;
+    d0 += __builtin_popcountll(__ballot(d < A && !own));
+    nlong += __builtin_popcountll(__ballot(own && c_end(pl.pref_end[off + d]) - (C + 1) > kLongSum));
+  }
   auto src = [&](const float* base, int64_t c, int d, int q) { return base + c * cstride + static_cast<int64_t>(d) * 2 * D + 4 * q; };
   auto finish = [&](int d, int q, float (&v)[4]) {
     const int tv = q / (D / 4);
@@ -1722,20 +1729,19 @@ __global__ __launch_bounds__(kCarryThreads) void bwd_carry_kernel(
   };
   // Long sums: (entry, 64 jobs) units.
   const int nqb = (Q + 63) / 64;
-  const int wave = tid >> 6, lane = tid & 63;
+  const int wave = tid >> 6;
   for (int u = blockIdx.y; u < nlong * nqb; u += gridDim.y) {
     const int d = d0 + u / nqb;
     const int q = (u % nqb) * 64 + lane;
     const int c1 = c_end(pl.pref_end[off + d]);
     const int qc = min(q, Q - 1);  // lanes past a narrow row repeat its last job
-    float4 y[kFetch];
+    f4 y[kFetch];
     auto fetch = [&](int c) {  // this wave's chunks of the round from chunk c on, clamped
 #pragma unroll
       for (int x = 0; x < kFetch; ++x)
-        y[x] = *reinterpret_cast<const float4*>(src(E, min(c + wave * kFetch + x, c1 - 1), d, qc));
+        y[x] = *reinterpret_cast<const f4*>(src(E, min(c + wave * kFetch + x, c1 - 1), d, qc));
     };
-    float v[4];
-    load_vec<4>(src(F, C, d, qc), v);
+    f4 sum = *reinterpret_cast<const f4*>(src(F, C, d, qc));
     fetch(C + 1);
     for (int c = C + 1; c < c1; c += kRound) {
 #pragma unroll
@@ -1743,16 +1749,13 @@ __global__ __launch_bounds__(kCarryThreads) void bwd_carry_kernel(
       __syncthreads();
       if (c + kRound < c1) fetch(c + kRound);
       if (wave == 0)
-        for (int x = 0; x < min(kRound, c1 - c); ++x) {
-          const float4 e = part[x][lane];
-          v[0] += e.x;
-          v[1] += e.y;
-          v[2] += e.z;
-          v[3] += e.w;
-        }
+        for (int x = 0; x < min(kRound, c1 - c); ++x) sum += part[x][lane];
       __syncthreads();
     }
-    if (wave == 0 && q < Q) finish(d, q, v);
+    if (wave == 0 && q < Q) {
+      float v[4] = {sum[0], sum[1], sum[2], sum[3]};
+      finish(d, q, v);
+    }
   }
   const int jobs = (A - d0 - nlong) * Q;
   for (int j = blockIdx.y * kCarryThreads + tid; j < jobs; j += gridDim.y * kCarryThreads) {

@@ -1,0 +1,61 @@
+"""What the compiled kernels must keep, read from the built library's gfx950
+code objects: a kernel whose working set is meant to stay in registers has no
+scratch."""
+from __future__ import annotations
+
+import struct
+import subprocess
+
+import pytest
+
+from agpt_amd import _native, build
+
+LLVM = "/opt/rocm/llvm/bin/"
+MAGIC = b"__CLANG_OFFLOAD_BUNDLE__"
+
+
+def _code_objects():
+    """The gfx950 ELF images embedded in the library, one per source file."""
+    data = (build.LIB / "libagpt_attn.so").read_bytes()
+    at = data.find(MAGIC)
+    while at >= 0:
+        n, = struct.unpack_from("<Q", data, at + len(MAGIC))
+        pos = at + len(MAGIC) + 8
+        for _ in range(n):
+            off, size, name_len = struct.unpack_from("<QQQ", data, pos)
+            name = data[pos + 24:pos + 24 + name_len]
+            pos += 24 + name_len
+            if b"gfx950" in name and size:
+                yield data[at + off:at + off + size]
+        at = data.find(MAGIC, pos)
+
+
+@pytest.fixture(scope="module")
+def images(tmp_path_factory):
+    _native.attn_lib()
+    out = []
+    for i, img in enumerate(_code_objects()):
+        p = tmp_path_factory.mktemp("co") / f"{i}.elf"
+        p.write_bytes(img)
+        out.append(str(p))
+    assert len(out) == len(build.HIP_SOURCES)
+    return out
+
+
+def _kernels(images, part):
+    """(name, scratch bytes per lane) of the kernels whose name holds `part`."""
+    found = []
+    for img in images:
+        notes = subprocess.run([LLVM + "llvm-readelf", "--notes", img], capture_output=True, text=True, check=True).stdout
+        for kernel in notes.split("  - .agpr_count:")[1:]:
+            field = lambda key: kernel.split(f".{key}:")[1].split()[0]
+            if part in field("name"):
+                found.append((field("name"), int(field("private_segment_fixed_size"))))
+    return found
+
+
+def test_carry_reduction_uses_no_scratch(images):
+    found = _kernels(images, "bwd_carry_kernel")
+    assert len(found) == 3  # head dims 16, 32, 64
+    for name, scratch in found:
+        assert scratch == 0, f"{name}: {scratch} bytes of scratch per lane"
