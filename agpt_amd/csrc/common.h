@@ -128,6 +128,12 @@ __device__ __forceinline__ void rope_inverse(float (&x)[HD], const float* __rest
   }
 }
 
+// The workgroup's number. (Without IEEE mode the device library's helpers
+// behind blockIdx and gridDim are not inlined: each use is a call, which waits
+// for every load in flight. A grid size comes as a kernel argument.)
+__device__ __forceinline__ int block_x() { return static_cast<int>(__builtin_amdgcn_workgroup_id_x()); }
+__device__ __forceinline__ int block_y() { return static_cast<int>(__builtin_amdgcn_workgroup_id_y()); }
+
 __device__ __forceinline__ float fast_exp2(float x) { return __builtin_amdgcn_exp2f(x); }
 __device__ __forceinline__ float fast_log2(float x) { return __builtin_amdgcn_logf(x); }
 

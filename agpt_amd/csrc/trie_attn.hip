@@ -90,6 +90,7 @@ struct PlanDev {
   int32_t chunk_tiles;
   int32_t n_chunks;
   int32_t n_prefix;  // pref_off[n_tiles]
+  int32_t grid;      // workgroups of this launch (block kernels), or along y
   // Deep query side: the tile of claim i is tile_order[i] (tiles of more key
   // chunks first, DFS order within), or tile i when null.
   const int32_t* tile_order;
@@ -428,7 +429,7 @@ __global__ __launch_bounds__(256) void trie_bwd_chunk_kernel(PlanDev pl, const f
                                                              const float* __restrict__ Pv,
                                                              float* __restrict__ Ck,
                                                              float* __restrict__ Cv, int D) {
-  const int c = blockIdx.x;
+  const int c = block_x();
   const int u0 = c * kChunkTiles;
   const int nu = min(pl.n_tiles - u0, kChunkTiles);
   __shared__ int offs[kChunkTiles + 1];
@@ -443,7 +444,7 @@ __global__ __launch_bounds__(256) void trie_bwd_chunk_kernel(PlanDev pl, const f
   __syncthreads();
   const int Q = D / 4;
   const int total = 2 * min_a * Q;  // (slot, K or V, 4 columns)
-  for (int idx = blockIdx.y * blockDim.x + threadIdx.x; idx < total; idx += gridDim.y * blockDim.x) {
+  for (int idx = block_y() * 256 + threadIdx.x; idx < total; idx += pl.grid * 256) {
     const int k = idx / (2 * Q);
     const int tv = (idx - k * 2 * Q) / Q;
     const int col = (idx % Q) * 4;
@@ -844,8 +845,9 @@ struct Arena {
 
 bool head_dim_supported(int hd) { return hd == 4 || hd == 8 || hd == 16 || hd == 32 || hd == 64; }
 
-PlanDev plan_dev(const agpt_attn_s* h) {
+PlanDev plan_dev(const agpt_attn_s* h, int grid = 0) {
   PlanDev p;
+  p.grid = grid;
   p.parent = h->d_parent;
   p.depth = h->d_depth;
   p.end = h->d_end;
@@ -1848,7 +1850,7 @@ void launch_fwd(const agpt_attn_s* h, const void* q, const void* k, const void* 
           const int grid = stream_grid(h, fn, h->fwd_lds);
           clear_sched_past(h, grid, HG, st);
           hipLaunchKernelGGL(fn, dim3(grid), dim3(agpt_blk::kThreads), h->fwd_lds,
-                             st, plan_dev(h), static_cast<const Tin*>(q), static_cast<const Tin*>(k),
+                             st, plan_dev(h, grid), static_cast<const Tin*>(q), static_cast<const Tin*>(k),
                              static_cast<const Tin*>(v), static_cast<Tin*>(o), lse, h->cfg.n_heads, scale);
         }
       });
@@ -1899,7 +1901,7 @@ void launch_carry(const agpt_attn_s* h, float* dk, float* dv, const float* acc_d
   const int jobs = agpt_blk::prefix_cap(h->max_depth) * h->cfg.n_heads * HD / 2;
   const int split = std::max(1, std::min((jobs + agpt_blk::kCarryThreads - 1) / agpt_blk::kCarryThreads, (2048 + n - 1) / n));
   hipLaunchKernelGGL((agpt_blk::bwd_carry_kernel<HD, PlanDev, RopeArgs>), dim3(n, split), dim3(agpt_blk::kCarryThreads),
-                     0, st, plan_dev(h), h->d_E, h->d_F, dk, dv, acc_dk, acc_dv, rope, h->cfg.n_heads);
+                     0, st, plan_dev(h, split), h->d_E, h->d_F, dk, dv, acc_dk, acc_dv, rope, h->cfg.n_heads);
 }
 
 template <int HD, typename Tin>
@@ -1925,7 +1927,7 @@ void launch_bwd(const agpt_attn_s* h, const void* q, const void* k, const void* 
           const int grid = stream_grid(h, fb, lds, HG);
           clear_sched_past(h, grid, HG, st);
           hipLaunchKernelGGL(fb, dim3(grid), dim3(agpt_blk::kThreads), lds,
-                             st, plan_dev(h), static_cast<const Tin*>(q), static_cast<const Tin*>(k),
+                             st, plan_dev(h, grid), static_cast<const Tin*>(q), static_cast<const Tin*>(k),
                              static_cast<const Tin*>(v), static_cast<const Tin*>(o), lse,
                              static_cast<const Tin*>(dO), dq, dk, dv, kCarry ? h->d_E : h->d_Pk,
                              kCarry ? h->d_F : h->d_Pv, acc_dk, acc_dv, rope, h->cfg.n_heads, scale);
@@ -2074,12 +2076,12 @@ void launch_bwd(const agpt_attn_s* h, const void* q, const void* k, const void* 
           const int q_grid = stream_grid(h, fq, q_lds), kv_grid = stream_grid(h, fk, kv_lds);
           clear_sched_past(h, std::min(q_grid, kv_grid), HG, st);
           hipLaunchKernelGGL(fq, dim3(q_grid), dim3(agpt_blk::kThreads), q_lds,
-                             st, plan_dev(h), static_cast<const Tin*>(q), static_cast<const Tin*>(k),
+                             st, plan_dev(h, q_grid), static_cast<const Tin*>(q), static_cast<const Tin*>(k),
                              static_cast<const Tin*>(v), static_cast<const Tin*>(o), lse,
                              static_cast<const Tin*>(dO), dq, h->d_Dl, rope, h->cfg.n_heads, scale);
           pm.mark(1);
           hipLaunchKernelGGL(fk, dim3(kv_grid), dim3(agpt_blk::kThreads), kv_lds,
-                             st, plan_dev(h), static_cast<const Tin*>(q), static_cast<const Tin*>(k),
+                             st, plan_dev(h, kv_grid), static_cast<const Tin*>(q), static_cast<const Tin*>(k),
                              static_cast<const Tin*>(v), lse, h->d_Dl, static_cast<const Tin*>(dO), dk, dv,
                              h->d_Pk, h->d_Pv, acc_dk, acc_dv, rope, h->cfg.n_heads, scale);
         }
@@ -2114,7 +2116,7 @@ void launch_bwd(const agpt_attn_s* h, const void* q, const void* k, const void* 
   pm.mark(2);
   if (h->n_tiles > 1) {
     const int split = std::max(1, std::min((h->max_depth * D / 2 + 255) / 256, (2048 + h->n_chunks - 1) / h->n_chunks));
-    hipLaunchKernelGGL(trie_bwd_chunk_kernel, dim3(h->n_chunks, split), dim3(256), 0, st, plan_dev(h), h->d_Pk,
+    hipLaunchKernelGGL(trie_bwd_chunk_kernel, dim3(h->n_chunks, split), dim3(256), 0, st, plan_dev(h, split), h->d_Pk,
                        h->d_Pv, h->d_Ck, h->d_Cv, D);
     pm.mark(3);
     auto reduce = [&](auto vw) {

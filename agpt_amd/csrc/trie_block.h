@@ -603,7 +603,7 @@ struct BStream {
 // Dynamic tile chunks. Workgroups claim (chunk, head group) pairs (chunk c =
 // tiles [cK, (c+1)K), the last chunk running to the end): workgroup b starts
 // on claim b, further claims come from one counter per kernel, cleared
-// before the launch, counted on from the grid size. Where the grid covers
+// before the launch, counted on from the grid size (plan.grid). Where the grid covers
 // every claim no counter is read, nor cleared by a launch of its own (see
 // clear_sched_past). A workgroup claims its next chunk during the current one, so with three or more tiles per
 // chunk the claim is known before the last tile's prefetch; within a chunk
@@ -613,6 +613,7 @@ struct BStream {
 template <typename PlanT>
 struct ChunkLoop {
   int* ctr;
+  const PlanT& plan;
   int nch, ngr, K, ntiles;
   int t, tend, hg, nxt, nxt_c, nt, gr, phase;
   bool sent, known;  // the next claim is sent / published
@@ -624,11 +625,12 @@ struct ChunkLoop {
   __device__ __forceinline__ bool valid(int c) const { return chunk_of(c) < nch; }
 
   __device__ __forceinline__ ChunkLoop(const PlanT& pl, int* ctr_, int ngr_)
-      : ctr(ctr_), nch(pl.n_chunks), ngr(ngr_), K(pl.chunk_tiles), ntiles(pl.n_tiles) {
+      : ctr(ctr_), plan(pl), nch(pl.n_chunks), ngr(ngr_), K(pl.chunk_tiles), ntiles(pl.n_tiles) {
     // The block's number through an opaque move: with the claim visible to
     // the compiler it hoists the tiles' address arithmetic out of the loop
-    // (the one-pass backward 224 -> 253 VGPRs, 28 spilled at head_dim 32).
-    int c = static_cast<int>(blockIdx.x);
+    // (the one-pass backward 226 -> 253 VGPRs, 28 spilled at head_dim 32,
+    // where one stays, stored and reloaded once a tile).
+    int c = block_x();
     asm volatile("" : "+v"(c));
     c = uniform(c);
     hg = c % ngr;
@@ -642,8 +644,7 @@ struct ChunkLoop {
   }
   // The next claim (one lane's; past the last one where the grid covers all).
   __device__ __forceinline__ int claim() {
-    const int n = static_cast<int>(gridDim.x);
-    return n < nch * ngr ? n + atomicAdd(ctr, 1) : n;
+    return plan.grid < nch * ngr ? plan.grid + atomicAdd(ctr, 1) : plan.grid;
   }
   __device__ __forceinline__ int cend(int ch) const { return ch == nch - 1 ? ntiles : (ch + 1) * K; }
 
@@ -1687,7 +1688,7 @@ __global__ __launch_bounds__(kCarryThreads) void bwd_carry_kernel(
   constexpr int kFetch = 4;                            // chunks a wave fetches per round of a long sum
   constexpr int kRound = kFetch * kCarryThreads / 64;  // chunks per round
   __shared__ f4 part[kRound][64];
-  const int C = blockIdx.x;
+  const int C = block_x();
   const int K = pl.chunk_tiles;
   const int64_t rows_per_chunk = static_cast<int64_t>(K) * kTile;
   const int64_t sC = C * rows_per_chunk;
@@ -1730,7 +1731,7 @@ __global__ __launch_bounds__(kCarryThreads) void bwd_carry_kernel(
   // Long sums: (entry, 64 jobs) units.
   const int nqb = (Q + 63) / 64;
   const int wave = tid >> 6;
-  for (int u = blockIdx.y; u < nlong * nqb; u += gridDim.y) {
+  for (int u = block_y(); u < nlong * nqb; u += pl.grid) {
     const int d = d0 + u / nqb;
     const int q = (u % nqb) * 64 + lane;
     const int c1 = c_end(pl.pref_end[off + d]);
@@ -1758,7 +1759,7 @@ __global__ __launch_bounds__(kCarryThreads) void bwd_carry_kernel(
     }
   }
   const int jobs = (A - d0 - nlong) * Q;
-  for (int j = blockIdx.y * kCarryThreads + tid; j < jobs; j += gridDim.y * kCarryThreads) {
+  for (int j = block_y() * kCarryThreads + tid; j < jobs; j += pl.grid * kCarryThreads) {
     const int d = d0 + nlong + j / Q;
     const int q = j % Q;
     float v[4];

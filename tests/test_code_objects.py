@@ -1,6 +1,7 @@
 """What the compiled kernels must keep, read from the built library's gfx950
 code objects: a kernel whose working set is meant to stay in registers has no
-scratch."""
+scratch, and the block kernels' loops hold no function call (a call waits for
+every load in flight)."""
 from __future__ import annotations
 
 import struct
@@ -59,3 +60,28 @@ def test_carry_reduction_uses_no_scratch(images):
     assert len(found) == 3  # head dims 16, 32, 64
     for name, scratch in found:
         assert scratch == 0, f"{name}: {scratch} bytes of scratch per lane"
+
+
+def test_block_kernels_call_at_most_the_thread_number(images):
+    """The block kernels and the reductions behind them: one call, the thread's
+    number at the kernel's start. The workgroup's number and the grid size are
+    read without."""
+    names = ("agpt_blk10fwd_kernel", "agpt_blk12bwd_q_kernel", "agpt_blk13bwd_kv_kernel", "agpt_blk10bwd_kernel",
+             "agpt_blk16bwd_carry_kernel", "21trie_bwd_chunk_kernel")
+    calls: dict = {}
+    for img in images:
+        text = subprocess.run([LLVM + "llvm-objdump", "-d", "--no-show-raw-insn", "--no-leading-addr", img],
+                              capture_output=True, text=True, check=True).stdout
+        cur = None
+        for line in text.splitlines():
+            if line.endswith(">:"):
+                cur = line.split("<")[-1][:-2]
+                if any(n in cur for n in names):
+                    calls[cur] = 0
+                else:
+                    cur = None
+            elif cur and "s_swappc_b64" in line:
+                calls[cur] += 1
+    assert {n for n in names if any(n in k for k in calls)} == set(names)
+    for name, n in calls.items():
+        assert n <= 1, f"{name}: {n} calls"
