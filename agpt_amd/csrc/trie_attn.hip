@@ -728,6 +728,8 @@ struct agpt_attn_s {
   int fhg = 1;                  // heads per workgroup of the one-pass backward
   bool carry = false;           // one-pass backward carries path sums (E, F replace Pk, Pv)
   bool rope_lds = false;        // block backward: the rotations fit in LDS at the same workgroups per CU
+  bool rope_lds_q = false;      // the same of the deep dQ kernel
+  bool rope_lds_kv = false;     // and of the deep carry key side
   bool deep = false;            // block kernels at head_dim 64: streamed key set (trie_deep.h)
   bool deep_carry = false;      // deep key side carries path sums (E, F replace Pk, Pv)
   bool dq_one_pass = true;      // deep bf16 dQ kernel: δ and dQ in one pass over the keys
@@ -1003,6 +1005,7 @@ namespace {
 // chain groups hold up to QB queries / KB keys (at most four).
 // AGPT_ATTN_VARIANT / _HG / _TILE / _QB / _KB override (tuning).
 void fit_scratch(agpt_attn_s* h);
+void fit_deep_rope(agpt_attn_s* h);
 
 void choose_variant(agpt_attn_s* h, int& tile) {
   const int hd = h->cfg.head_dim, H = h->cfg.n_heads;
@@ -1444,6 +1447,7 @@ int plan_impl(agpt_attn_s* h, const int32_t* ext, int64_t n_ext, int32_t A0,
                      "agpt_attn_plan_static: the batch needs %zu bytes of device tables and workspace, more "
                      "than the %zu bytes of static scratch (AGPT_STATIC_SCRATCH_BYTES); use agpt_attn_plan",
                      ar.used, kScratchBytes);
+  fit_deep_rope(h);
   h->planned = true;
   g_last_error.clear();
   return AGPT_OK;
@@ -1607,12 +1611,12 @@ extern "C" const char* agpt_attn_describe(agpt_attn_handle h) {
   else if (h->variant == 6 && h->deep)
     snprintf(buf, sizeof(buf),
              "streamed key ring (deep prefixes) 16x16 mfma, split backward%s: tile_rows=%d tiles=%d "
-             "heads_per_wg=1 key_chunk=%d fwd_lds=%zu bwd_q_lds=%zu bwd_kv_lds=%zu lds_limit=%d",
+             "heads_per_wg=1 key_chunk=%d fwd_lds=%zu bwd_q_lds=%zu bwd_kv_lds=%zu rope_in_lds=%d/%d lds_limit=%d",
              h->deep_range ? " with the key side by subtree range"
              : h->deep_carry ? " with path-carry"
                              : "",
              h->tile, h->n_tiles, agpt_deep::kChunk, h->fwd_lds, h->bq_lds,
-             h->kv_lds, h->max_lds);
+             h->kv_lds, h->rope_lds_q, h->rope_lds_kv, h->max_lds);
   else if (h->variant == 6)
     snprintf(buf, sizeof(buf),
              "streaming block-sparse 16x16 mfma, %s backward: tile_rows=%d tiles=%d heads_per_wg=%d "
@@ -1801,18 +1805,48 @@ void with_block_heads(const agpt_attn_s* h, int uh, Fn&& fn) {
   });
 }
 
-// Deep kernels: puts the rotations of every depth in `fn`'s LDS (see
-// choose_variant) when that keeps its workgroups per CU; returns the bytes.
-// 596K rows of 4 x 64, depth 32, with the carry kernel's two turns: fp32 dQ
-// kernel 1.01 -> 0.89 ms, key side 1.62 -> 1.51; bf16 key side 1.01 -> 0.73.
-template <typename Fn>
-size_t stage_rope(const agpt_attn_s* h, Fn fn, size_t lds, int hd, RopeArgs& rope) {
-  const size_t extra = agpt_blk::rope_lds_bytes(h->max_depth, hd);
-  if (!rope.cos_t || env_int("AGPT_ATTN_ROPELDS", 1) == 0) return 0;
-  set_lds(fn, lds + extra);
-  if (wg_per_cu(fn, lds + extra, h->max_lds) < std::max(1, wg_per_cu(fn, lds, h->max_lds))) return 0;
-  rope.lds_rows = h->max_depth;
-  return extra;
+// The carry key side's kernel and its LDS without rotations. Key slots of a
+// tile: prefix_cap + 64. A plan to depth 129 keeps every slot's sums in
+// registers (2 turns of 4 blocks of 16 to depth 65, else 3) and, in bf16, each
+// slot's K/V slices in an LDS cache tagged by row; deeper plans (or
+// AGPT_ATTN_REGITERS=2) keep the first 4 kRegItersDeep blocks in registers and
+// the rest in the carry rows.
+template <int HD, typename Tin, typename Fn>
+auto with_carry_kernel(const agpt_attn_s* h, Fn&& fn) {
+  const bool regs = env_int("AGPT_ATTN_REGCARRY", 1) != 0;
+  const int slots = agpt_blk::prefix_cap(h->max_depth) + agpt_deep::kTile;
+  const int iters = env_int("AGPT_ATTN_REGITERS", 0);  // 0: by depth
+  const bool all2 = slots <= 64 * agpt_deep::kRegItersDeep && iters == 0;
+  const bool all3 = slots <= 64 * agpt_deep::kRegIters && !all2 && (iters == 0 || iters == agpt_deep::kRegIters);
+  auto fc = !regs  ? agpt_deep::bwd_kv_carry_kernel<HD, Tin, 0, false, PlanDev, RopeArgs>
+            : all2 ? agpt_deep::bwd_kv_carry_kernel<HD, Tin, agpt_deep::kRegItersDeep, true, PlanDev, RopeArgs>
+            : all3 ? agpt_deep::bwd_kv_carry_kernel<HD, Tin, agpt_deep::kRegIters, true, PlanDev, RopeArgs>
+                   : agpt_deep::bwd_kv_carry_kernel<HD, Tin, agpt_deep::kRegItersDeep, false, PlanDev, RopeArgs>;
+  return fn(fc, h->kv_lds + agpt_deep::kv_cache_bytes(all2 ? agpt_deep::kRegItersDeep : agpt_deep::kRegIters,
+                                                      regs && (all2 || all3), sizeof(Tin)));
+}
+
+// Deep kernels: whether the rotations of every depth go into LDS (see
+// choose_variant), decided once per plan: where that keeps the workgroups per
+// CU. 596K rows of 4 x 64, depth 32, with the carry kernel's two turns: fp32
+// dQ kernel 1.01 -> 0.89 ms, key side 1.62 -> 1.51; bf16 key side 1.01 -> 0.73.
+template <typename Tin>
+void fit_deep_rope_t(agpt_attn_s* h) {
+  auto keeps = [&](auto fn, size_t lds) {
+    const size_t with = lds + agpt_blk::rope_lds_bytes(h->max_depth, 64);
+    set_lds(fn, with);
+    return wg_per_cu(fn, with, h->max_lds) >= std::max(1, wg_per_cu(fn, lds, h->max_lds));
+  };
+  if constexpr (sizeof(Tin) == 4) h->rope_lds_q = keeps(agpt_deep::bwd_q_kernel<64, Tin, PlanDev, RopeArgs, false>, h->bq_lds);
+  if (h->deep_carry) h->rope_lds_kv = with_carry_kernel<64, Tin>(h, keeps);
+}
+
+void fit_deep_rope(agpt_attn_s* h) {
+  h->rope_lds_q = h->rope_lds_kv = false;
+  if (h->variant != 6 || !h->deep || h->chain_plan || env_int("AGPT_ATTN_ROPELDS", 1) == 0) return;
+  if (h->cfg.dtype == AGPT_DTYPE_F32) fit_deep_rope_t<float>(h);
+  else fit_deep_rope_t<bf16_t>(h);
+  (void)hipGetLastError();  // a failed probe only leaves the table out
 }
 
 template <int HD, typename Tin>
@@ -1989,9 +2023,10 @@ void launch_bwd(const agpt_attn_s* h, const void* q, const void* k, const void* 
       clear_sched(h, st);
       const int hpu = deep_heads_per_unit(h);
       auto launch_q = [&](auto fq) {
-        set_lds(fq, h->bq_lds);
         RopeArgs rope_q = rope;
-        const size_t lds = h->bq_lds + (sizeof(Tin) == 4 ? stage_rope(h, fq, h->bq_lds, HD, rope_q) : 0);
+        rope_q.lds_rows = rope.cos_t && h->rope_lds_q ? h->max_depth : 0;
+        const size_t lds = h->bq_lds + agpt_blk::rope_lds_bytes(rope_q.lds_rows, HD);
+        set_lds(fq, lds);
         hipLaunchKernelGGL(fq, dim3(stream_grid(h, fq, lds, hpu)), dim3(agpt_deep::kThreads), lds, st,
                            plan_dev(h), static_cast<const Tin*>(q), static_cast<const Tin*>(k),
                            static_cast<const Tin*>(v), static_cast<const Tin*>(o), lse,
@@ -2023,32 +2058,19 @@ void launch_bwd(const agpt_attn_s* h, const void* q, const void* k, const void* 
         return;
       }
       if (h->deep_carry) {
-        // Key slots of a tile: prefix_cap + 64. A plan to depth 128 keeps
-        // every slot's sums in registers (2 turns of 4 blocks of 16 to depth
-        // 65, else 3) and, in bf16, each slot's K/V slices in an LDS cache
-        // tagged by row; deeper plans (or AGPT_ATTN_REGITERS=2) keep the first
-        // 4 kRegItersDeep blocks in registers and the rest in the carry rows.
-        const bool regs = env_int("AGPT_ATTN_REGCARRY", 1) != 0;
-        const int slots = agpt_blk::prefix_cap(h->max_depth) + agpt_deep::kTile;
-        const int iters = env_int("AGPT_ATTN_REGITERS", 0);  // 0: by depth
-        const bool all2 = slots <= 64 * agpt_deep::kRegItersDeep && iters == 0;
-        const bool all3 = slots <= 64 * agpt_deep::kRegIters && !all2 && (iters == 0 || iters == agpt_deep::kRegIters);
-        auto fc = !regs  ? agpt_deep::bwd_kv_carry_kernel<HD, Tin, 0, false, PlanDev, RopeArgs>
-                  : all2 ? agpt_deep::bwd_kv_carry_kernel<HD, Tin, agpt_deep::kRegItersDeep, true, PlanDev, RopeArgs>
-                  : all3 ? agpt_deep::bwd_kv_carry_kernel<HD, Tin, agpt_deep::kRegIters, true, PlanDev, RopeArgs>
-                         : agpt_deep::bwd_kv_carry_kernel<HD, Tin, agpt_deep::kRegItersDeep, false, PlanDev, RopeArgs>;
-        size_t lds = h->kv_lds + agpt_deep::kv_cache_bytes(all2 ? agpt_deep::kRegItersDeep : agpt_deep::kRegIters,
-                                                           regs && (all2 || all3), sizeof(Tin));
-        RopeArgs rope_kv = rope;
-        lds += stage_rope(h, fc, lds, HD, rope_kv);
-        set_lds(fc, lds);
-        int cus = 256;
-        (void)hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, h->device);
-        const int grid = std::max(1, std::min(wg_per_cu(fc, lds, h->max_lds) * cus, h->cs_slots));
-        hipLaunchKernelGGL(fc, dim3(grid), dim3(agpt_deep::kThreads), lds, st, plan_dev(h),
-                           static_cast<const Tin*>(q), static_cast<const Tin*>(k), static_cast<const Tin*>(v), lse,
-                           h->d_Dl, static_cast<const Tin*>(dO), dk, dv, h->d_E, h->d_F, h->d_Cs, acc_dk, acc_dv,
-                           rope_kv, h->cfg.n_heads, scale);
+        with_carry_kernel<HD, Tin>(h, [&](auto fc, size_t lds) {
+          RopeArgs rope_kv = rope;
+          rope_kv.lds_rows = rope.cos_t && h->rope_lds_kv ? h->max_depth : 0;
+          lds += agpt_blk::rope_lds_bytes(rope_kv.lds_rows, HD);
+          set_lds(fc, lds);
+          int cus = 256;
+          (void)hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, h->device);
+          const int grid = std::max(1, std::min(wg_per_cu(fc, lds, h->max_lds) * cus, h->cs_slots));
+          hipLaunchKernelGGL(fc, dim3(grid), dim3(agpt_deep::kThreads), lds, st, plan_dev(h),
+                             static_cast<const Tin*>(q), static_cast<const Tin*>(k), static_cast<const Tin*>(v), lse,
+                             h->d_Dl, static_cast<const Tin*>(dO), dk, dv, h->d_E, h->d_F, h->d_Cs, acc_dk, acc_dv,
+                             rope_kv, h->cfg.n_heads, scale);
+        });
         pm.mark(2);
         pm.mark(3);
         launch_carry<HD>(h, dk, dv, acc_dk, acc_dv, rope, st);

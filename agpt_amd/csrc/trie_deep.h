@@ -64,7 +64,7 @@ constexpr int kKeyCap = (kMaxDepth - 1 + kTile + kChunk - 1) / kChunk * kChunk;
 // in kRegItersDeep blocks per wave for plans to depth 65, in kRegIters for
 // plans to depth kRegDepth; deeper plans keep their first kRegItersDeep.
 constexpr int kRegIters = 3;
-constexpr int kRegDepth = 4 * kRegIters * 16 - kTile;  // 128
+constexpr int kRegDepth = 4 * kRegIters * 16 - kTile + 1;  // 129
 constexpr int kRegItersDeep = 2;
 // Running max of a query before it has seen a key: finite, so that exp2 of
 // a masked score (-inf) minus it is 0, never NaN.

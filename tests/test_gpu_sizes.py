@@ -143,11 +143,11 @@ def _rooted(rows, depth, seed):
 
 
 @pytest.mark.parametrize("dtype", ["f32", "bf16"])
-@pytest.mark.parametrize("depth,chunk,iters", [(64, 2, 0), (65, 3, 0), (66, 2, 0), (128, 3, 0), (129, 2, 0), (60, 2, 3),
-                                               (65, 2, 2), (128, 2, 2)])
+@pytest.mark.parametrize("depth,chunk,iters", [(64, 2, 0), (65, 3, 0), (66, 2, 0), (128, 3, 0), (129, 2, 0), (134, 2, 0),
+                                               (60, 2, 3), (65, 2, 2), (128, 2, 2)])
 def test_deep_carry_register_turns(gpu, monkeypatch, dtype, depth, chunk, iters):
     """The deep key side's path carry on both sides of its register rules: two
-    turns of four key blocks to depth 65, three to depth 128, past that the
+    turns of four key blocks to depth 65, three to depth 129, past that the
     first slots only; three turns on a shallow plan and two on a deep one by
     the knob. A root over ten tiles and more keeps the subtree-range kernel
     out."""
@@ -158,7 +158,7 @@ def test_deep_carry_register_turns(gpu, monkeypatch, dtype, depth, chunk, iters)
 
 
 @pytest.mark.parametrize("dtype", ["f32", "bf16"])
-@pytest.mark.parametrize("depth", [20, 65, 72, 129])
+@pytest.mark.parametrize("depth", [20, 65, 72, 129, 134])
 def test_rope_table_in_lds_deep(gpu, monkeypatch, dtype, depth):
     """Head dim 64: the deep kernels' rotations from LDS (the fp32 dQ kernel,
     both carry kernels) give the bytes of the caller's 64-row tables."""
@@ -172,6 +172,25 @@ def test_rope_table_in_lds_deep(gpu, monkeypatch, dtype, depth):
         res.append(run_gpu(par, Q, K, V, G, 2, 64, dtype, rope=ORC.rope_table(64, 64)))
     for name, a, b in zip(("O", "lse", "dQ", "dK", "dV"), *res):
         np.testing.assert_array_equal(a, b, err_msg=name)
+
+
+@pytest.mark.parametrize("dtype,depth,want", [("f32", 20, "1/1"), ("f32", 134, "0/1"), ("bf16", 20, "0/1"), ("bf16", 65, "0/1"),
+                                              ("bf16", 129, "0/0"), ("bf16", 134, "0/1")])
+def test_deep_rotations_are_placed_by_the_plan(gpu, monkeypatch, dtype, depth, want):
+    """Head dim 64: the plan decides once which kernels (dQ / key side) take
+    the rotations from LDS: those whose workgroups per CU it leaves alone (the
+    bf16 key side's cache from depth 66 to 129 does not). The knob is read there too."""
+    import torch
+
+    from agpt_amd.attention import TrieAttention
+    monkeypatch.setenv("AGPT_ATTN_CHUNK", "2")
+    par = _rooted(11 * 64 + 5, depth, seed=depth)
+    for knob, expect in (("1", want), ("0", "0/0")):
+        monkeypatch.setenv("AGPT_ATTN_ROPELDS", knob)
+        att = TrieAttention(2, 64, max_depth=depth, dtype=torch.float32 if dtype == "f32" else torch.bfloat16)
+        att.plan(par)
+        assert f"rope_in_lds={expect} " in att.describe()
+        att.close()
 
 
 @pytest.mark.parametrize("H,hd,dtype", [(8, 16, "f32"), (4, 32, "f32"), (2, 64, "f32"), (2, 64, "bf16")])
