@@ -603,7 +603,7 @@ struct BStream {
 // Dynamic tile chunks. Workgroups claim (chunk, head group) pairs (chunk c =
 // tiles [cK, (c+1)K), the last chunk running to the end): workgroup b starts
 // on claim b, further claims come from one counter per kernel, cleared
-// before the launch, counted on from the grid size (plan.grid). Where the grid covers
+// before the launch, counted on from the grid size. Where the grid covers
 // every claim no counter is read, nor cleared by a launch of its own (see
 // clear_sched_past). A workgroup claims its next chunk during the current one, so with three or more tiles per
 // chunk the claim is known before the last tile's prefetch; within a chunk
@@ -613,7 +613,6 @@ struct BStream {
 template <typename PlanT>
 struct ChunkLoop {
   int* ctr;
-  const PlanT& plan;
   int nch, ngr, K, ntiles;
   int t, tend, hg, nxt, nxt_c, nt, gr, phase;
   bool sent, known;  // the next claim is sent / published
@@ -625,11 +624,10 @@ struct ChunkLoop {
   __device__ __forceinline__ bool valid(int c) const { return chunk_of(c) < nch; }
 
   __device__ __forceinline__ ChunkLoop(const PlanT& pl, int* ctr_, int ngr_)
-      : ctr(ctr_), plan(pl), nch(pl.n_chunks), ngr(ngr_), K(pl.chunk_tiles), ntiles(pl.n_tiles) {
+      : ctr(ctr_), nch(pl.n_chunks), ngr(ngr_), K(pl.chunk_tiles), ntiles(pl.n_tiles) {
     // The block's number through an opaque move: with the claim visible to
     // the compiler it hoists the tiles' address arithmetic out of the loop
-    // (the one-pass backward 226 -> 253 VGPRs, 28 spilled at head_dim 32,
-    // where one stays, stored and reloaded once a tile).
+    // (the one-pass backward 226 -> 253 VGPRs, 28 spilled at head_dim 32).
     int c = block_x();
     asm volatile("" : "+v"(c));
     c = uniform(c);
@@ -644,7 +642,15 @@ struct ChunkLoop {
   }
   // The next claim (one lane's; past the last one where the grid covers all).
   __device__ __forceinline__ int claim() {
-    return plan.grid < nch * ngr ? plan.grid + atomicAdd(ctr, 1) : plan.grid;
+    // The grid size (the plan is every block kernel's first argument), read
+    // where it is needed: as plan.grid it is held in a register from the
+    // kernel's start, which displaces others in the tile loop (one VGPR of the
+    // head_dim 32 backward to scratch: 8 x 32, 807K rows 2,221 us for 2,167).
+    typedef const __attribute__((address_space(4))) PlanT* ArgsP;
+    ArgsP args = (ArgsP)__builtin_amdgcn_kernarg_segment_ptr();
+    asm volatile("" : "+s"(args));
+    const int n = args->grid;
+    return n < nch * ngr ? n + atomicAdd(ctr, 1) : n;
   }
   __device__ __forceinline__ int cend(int ch) const { return ch == nch - 1 ? ntiles : (ch + 1) * K; }
 

@@ -62,6 +62,16 @@ def test_carry_reduction_uses_no_scratch(images):
         assert scratch == 0, f"{name}: {scratch} bytes of scratch per lane"
 
 
+def test_block_kernels_use_no_scratch(images):
+    """The one-pass backward with the path carry sits at the register limit at
+    head_dim 32 (one head per workgroup)."""
+    found = _kernels(images, "agpt_blk10bwd_kernelILi32EfLi1ELb1E") + _kernels(images, "agpt_blk10bwd_kernelILi16E") + \
+        _kernels(images, "agpt_blk10fwd_kernel")
+    assert len(found) > 10
+    for name, scratch in found:
+        assert scratch == 0, f"{name}: {scratch} bytes of scratch per lane"
+
+
 def test_block_kernels_call_at_most_the_thread_number(images):
     """The block kernels and the reductions behind them: one call, the thread's
     number at the kernel's start. The workgroup's number and the grid size are
