@@ -1381,13 +1381,16 @@ int plan_impl(agpt_attn_s* h, const int32_t* ext, int64_t n_ext, int32_t A0,
     // per CU) still gets a claim: each chunk reads its first tile's prefix
     // from memory and writes E and F rows for the carry kernel. The deep key
     // side takes 2 at least where its per-tile partials (what chunks of one
-    // tile leave) are more than a static plan could hold: below that both
-    // plans keep the partials, and give the same bytes. Without a carry (the split block kernels) long chunks
-    // only save prefix reads: 4 at most. Forward + backward, 8 claims per CU
-    // and no floor against this rule: 31K rows of 8 x 64 bf16, depth 128, 1.67
-    // ms (chunks of 1) -> 0.30 (3); 767K of 4 x 32 1.91 (23) -> 1.69 (11);
-    // 744K of 8 x 64 bf16, depth 128, 3.83 (45) -> 3.68 (22); 90K of 8 x 16
-    // 0.207 (2) -> 0.197 (3); 891K of 8 x 16 bf16 1.59 (13) -> 1.38 (4).
+    // tile leave) are more than a static plan could hold; plans with chunks of
+    // one tile keep the partials as static plans do. Without a carry (the
+    // split block kernels) long chunks only save prefix reads: 4 at most.
+    // Forward + backward, 8 claims per CU and no floor against this rule: 31K
+    // rows of 8 x 64 bf16, depth 128, 1.67 ms (chunks of 1) -> 0.30 (3); 767K
+    // of 4 x 32 1.91 (23) -> 1.69 (11); 744K of 8 x 64 bf16, depth 128, 3.83
+    // (45) -> 3.68 (22); 90K of 8 x 16 0.207 (2) -> 0.197 (3); 891K of 8 x 16
+    // bf16 1.59 (13) -> 1.38 (4). The shorter chunks cost E and F: that deep
+    // plan takes 826 MiB at 22 tiles (backward 2,990 us, the carry kernel 105
+    // of them), 560 MiB at 45 (3,120 and 56), beside 8 GB of tensors.
     int cus = 256;
     (void)hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, h->device);
     cus = std::max(cus, 1);
@@ -1827,26 +1830,27 @@ auto with_carry_kernel(const agpt_attn_s* h, Fn&& fn) {
 }
 
 // Deep kernels: whether the rotations of every depth go into LDS (see
-// choose_variant), decided once per plan: where that keeps the workgroups per
-// CU. 596K rows of 4 x 64, depth 32, with the carry kernel's two turns: fp32
-// dQ kernel 1.01 -> 0.89 ms, key side 1.62 -> 1.51; bf16 key side 1.01 -> 0.73.
-template <typename Tin>
-void fit_deep_rope_t(agpt_attn_s* h) {
-  auto keeps = [&](auto fn, size_t lds) {
-    const size_t with = lds + agpt_blk::rope_lds_bytes(h->max_depth, 64);
-    set_lds(fn, with);
-    return wg_per_cu(fn, with, h->max_lds) >= std::max(1, wg_per_cu(fn, lds, h->max_lds));
-  };
-  if constexpr (sizeof(Tin) == 4) h->rope_lds_q = keeps(agpt_deep::bwd_q_kernel<64, Tin, PlanDev, RopeArgs, false>, h->bq_lds);
-  if (h->deep_carry) h->rope_lds_kv = with_carry_kernel<64, Tin>(h, keeps);
-}
-
+// choose_variant), decided once per plan and from sizes alone: where that
+// keeps the workgroups per CU (registers hold the dQ kernel and the register
+// carry to two, the carry rows' form to three). 596K rows of 4 x 64, depth 32,
+// with the carry kernel's two turns: fp32 dQ kernel 1.01 -> 0.89 ms, key side
+// 1.62 -> 1.51; bf16 key side 1.01 -> 0.73.
 void fit_deep_rope(agpt_attn_s* h) {
   h->rope_lds_q = h->rope_lds_kv = false;
   if (h->variant != 6 || !h->deep || h->chain_plan || env_int("AGPT_ATTN_ROPELDS", 1) == 0) return;
-  if (h->cfg.dtype == AGPT_DTYPE_F32) fit_deep_rope_t<float>(h);
-  else fit_deep_rope_t<bf16_t>(h);
-  (void)hipGetLastError();  // a failed probe only leaves the table out
+  auto keeps = [&](size_t lds, size_t tabs, size_t cap) {
+    auto per_cu = [&](size_t b) {
+      return std::min(cap, static_cast<size_t>(h->max_lds) / ((b + tabs + 511) & ~static_cast<size_t>(511)));
+    };
+    return per_cu(lds + agpt_blk::rope_lds_bytes(h->max_depth, 64)) >= std::max<size_t>(1, per_cu(lds));
+  };
+  const bool f32 = h->cfg.dtype == AGPT_DTYPE_F32;
+  h->rope_lds_q = f32 && keeps(h->bq_lds, sizeof(agpt_deep::KeyTables), 2);
+  auto carry = [&](auto, size_t lds) {
+    return keeps(lds, sizeof(agpt_deep::Tables), env_int("AGPT_ATTN_REGCARRY", 1) != 0 ? 2 : 3);
+  };
+  if (h->deep_carry)
+    h->rope_lds_kv = f32 ? with_carry_kernel<64, float>(h, carry) : with_carry_kernel<64, bf16_t>(h, carry);
 }
 
 template <int HD, typename Tin>
