@@ -609,9 +609,17 @@ struct BStream {
 // chunk the claim is known before the last tile's prefetch; within a chunk
 // the prefix moves LDS to LDS, the first tile of a chunk loads it from
 // memory. Results do not depend on which workgroup takes a tile.
+//
+// The grid size is read at the claim, from the plan as the kernel's first
+// argument: as plan.grid it stays in a register from the kernel's start, which
+// displaces others in the tile loop (one VGPR of the head_dim 32 backward to
+// scratch: 8 x 32, 807K rows 2,221 us for 2,167). kHeld: so all the same in
+// the head_dim 16 backward, where it spills nothing and the loop's schedule
+// comes out better (C2 backward 32.18 ms for 32.50).
 // ---------------------------------------------------------------------------
-template <typename PlanT>
+template <typename PlanT, bool kHeld = false>
 struct ChunkLoop {
+  const PlanT& plan;
   int* ctr;
   int nch, ngr, K, ntiles;
   int t, tend, hg, nxt, nxt_c, nt, gr, phase;
@@ -624,7 +632,7 @@ struct ChunkLoop {
   __device__ __forceinline__ bool valid(int c) const { return chunk_of(c) < nch; }
 
   __device__ __forceinline__ ChunkLoop(const PlanT& pl, int* ctr_, int ngr_)
-      : ctr(ctr_), nch(pl.n_chunks), ngr(ngr_), K(pl.chunk_tiles), ntiles(pl.n_tiles) {
+      : plan(pl), ctr(ctr_), nch(pl.n_chunks), ngr(ngr_), K(pl.chunk_tiles), ntiles(pl.n_tiles) {
     // The block's number through an opaque move: with the claim visible to
     // the compiler it hoists the tiles' address arithmetic out of the loop
     // (the one-pass backward 226 -> 253 VGPRs, 28 spilled at head_dim 32).
@@ -642,14 +650,15 @@ struct ChunkLoop {
   }
   // The next claim (one lane's; past the last one where the grid covers all).
   __device__ __forceinline__ int claim() {
-    // The grid size (the plan is every block kernel's first argument), read
-    // where it is needed: as plan.grid it is held in a register from the
-    // kernel's start, which displaces others in the tile loop (one VGPR of the
-    // head_dim 32 backward to scratch: 8 x 32, 807K rows 2,221 us for 2,167).
-    typedef const __attribute__((address_space(4))) PlanT* ArgsP;
-    ArgsP args = (ArgsP)__builtin_amdgcn_kernarg_segment_ptr();
-    asm volatile("" : "+s"(args));
-    const int n = args->grid;
+    int n;
+    if constexpr (kHeld) {
+      n = plan.grid;
+    } else {
+      typedef const __attribute__((address_space(4))) PlanT* ArgsP;
+      ArgsP args = (ArgsP)__builtin_amdgcn_kernarg_segment_ptr();
+      asm volatile("" : "+s"(args));
+      n = args->grid;
+    }
     return n < nch * ngr ? n + atomicAdd(ctr, 1) : n;
   }
   __device__ __forceinline__ int cend(int ch) const { return ch == nch - 1 ? ntiles : (ch + 1) * K; }
@@ -1238,7 +1247,7 @@ __global__ __launch_bounds__(kThreads, (kBwdWaves<HD, HG, kCarry>)) void bwd_ker
   constexpr int WS = ST::WS;
   __shared__ typename ST::Tables tb;
   extern __shared__ __align__(16) unsigned char dyn[];
-  ChunkLoop<PlanT> cl(pl, pl.sched + 1, H / HG);
+  ChunkLoop<PlanT, HD == 16> cl(pl, pl.sched + 1, H / HG);
   if (cl.t >= cl.ntiles) return;
   ST st(pl, K, V, Q, dO, O, lse, nullptr, H, 0, dyn, tb);
   st.dscale = scale;  // dS = P (dP - δ) scale, with V and δ taken times scale
