@@ -610,16 +610,15 @@ struct BStream {
 // the prefix moves LDS to LDS, the first tile of a chunk loads it from
 // memory. Results do not depend on which workgroup takes a tile.
 //
-// The grid size is read at the claim, from the plan as the kernel's first
-// argument: as plan.grid it stays in a register from the kernel's start, which
-// displaces others in the tile loop (one VGPR of the head_dim 32 backward to
-// scratch: 8 x 32, 807K rows 2,221 us for 2,167). kHeld: so all the same in
-// the head_dim 16 backward, where it spills nothing and the loop's schedule
-// comes out better (C2 backward 32.18 ms for 32.50).
+// The grid size is read where a claim is sent or learned, from the plan as the
+// kernel's first argument: as pl.grid it stays in a register from the kernel's
+// start, which displaces others in the tile loop (one VGPR of the head_dim 32
+// backward to scratch: 8 x 32, 807K rows 2,221 us for 2,167). It is added when
+// the claim is learned, as an add behind the atomic would wait for its result
+// (backward of 1.3K to 807K rows at ten head shapes 1.4 % longer).
 // ---------------------------------------------------------------------------
-template <typename PlanT, bool kHeld = false>
+template <typename PlanT>
 struct ChunkLoop {
-  const PlanT& plan;
   int* ctr;
   int nch, ngr, K, ntiles;
   int t, tend, hg, nxt, nxt_c, nt, gr, phase;
@@ -632,7 +631,7 @@ struct ChunkLoop {
   __device__ __forceinline__ bool valid(int c) const { return chunk_of(c) < nch; }
 
   __device__ __forceinline__ ChunkLoop(const PlanT& pl, int* ctr_, int ngr_)
-      : plan(pl), ctr(ctr_), nch(pl.n_chunks), ngr(ngr_), K(pl.chunk_tiles), ntiles(pl.n_tiles) {
+      : ctr(ctr_), nch(pl.n_chunks), ngr(ngr_), K(pl.chunk_tiles), ntiles(pl.n_tiles) {
     // The block's number through an opaque move: with the claim visible to
     // the compiler it hoists the tiles' address arithmetic out of the loop
     // (the one-pass backward 226 -> 253 VGPRs, 28 spilled at head_dim 32).
@@ -648,24 +647,23 @@ struct ChunkLoop {
     gr = 0;
     sent = known = false;
   }
-  // The next claim (one lane's; past the last one where the grid covers all).
-  __device__ __forceinline__ int claim() {
-    int n;
-    if constexpr (kHeld) {
-      n = plan.grid;
-    } else {
-      typedef const __attribute__((address_space(4))) PlanT* ArgsP;
-      ArgsP args = (ArgsP)__builtin_amdgcn_kernarg_segment_ptr();
-      asm volatile("" : "+s"(args));
-      n = args->grid;
-    }
-    return n < nch * ngr ? n + atomicAdd(ctr, 1) : n;
+  // Workgroups of the launch.
+  __device__ __forceinline__ int grid() const {
+    typedef const __attribute__((address_space(4))) PlanT* ArgsP;
+    ArgsP args = (ArgsP)__builtin_amdgcn_kernarg_segment_ptr();
+    asm volatile("" : "+s"(args));
+    return args->grid;
+  }
+  // Sends for the next claim (one lane), counted from the grid size on; where
+  // the grid covers every claim there is none, and grid() + 0 is past the last.
+  __device__ __forceinline__ void claim() {
+    if (grid() < nch * ngr) gr = atomicAdd(ctr, 1);
   }
   __device__ __forceinline__ int cend(int ch) const { return ch == nch - 1 ? ntiles : (ch + 1) * K; }
 
   template <typename ST>
   __device__ __forceinline__ void learn(ST& st) {
-    nxt_c = uniform(st.tb.grab);
+    nxt_c = grid() + uniform(st.tb.grab);
     nxt = valid(nxt_c) ? chunk_of(nxt_c) * K : -1;
     known = true;
   }
@@ -677,7 +675,7 @@ struct ChunkLoop {
   __device__ __forceinline__ void begin_tile(ST& st) {
     const bool within = t + 1 < tend;
     if (!within && !known) {
-      if (!sent && threadIdx.x == 0) gr = claim();
+      if (!sent && threadIdx.x == 0) claim();
       sent = true;
       if (threadIdx.x == 0) st.tb.grab = gr;
       __syncthreads();
@@ -695,7 +693,7 @@ struct ChunkLoop {
     if (nt < 0) return false;
     const bool cold = t + 1 >= tend;
     const bool pub = phase == 1 && !known;
-    if (!sent && threadIdx.x == 0) gr = claim();
+    if (!sent && threadIdx.x == 0) claim();
     sent = true;
     st.commit(cold, pub, gr);
     if (pub) learn(st);
@@ -1247,7 +1245,7 @@ __global__ __launch_bounds__(kThreads, (kBwdWaves<HD, HG, kCarry>)) void bwd_ker
   constexpr int WS = ST::WS;
   __shared__ typename ST::Tables tb;
   extern __shared__ __align__(16) unsigned char dyn[];
-  ChunkLoop<PlanT, HD == 16> cl(pl, pl.sched + 1, H / HG);
+  ChunkLoop<PlanT> cl(pl, pl.sched + 1, H / HG);
   if (cl.t >= cl.ntiles) return;
   ST st(pl, K, V, Q, dO, O, lse, nullptr, H, 0, dyn, tb);
   st.dscale = scale;  // dS = P (dP - δ) scale, with V and δ taken times scale

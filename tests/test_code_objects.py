@@ -72,26 +72,31 @@ def test_block_kernels_use_no_scratch(images):
         assert scratch == 0, f"{name}: {scratch} bytes of scratch per lane"
 
 
-def test_block_kernels_call_at_most_the_thread_number(images):
-    """The block kernels and the reductions behind them: one call, the thread's
-    number at the kernel's start. The workgroup's number and the grid size are
-    read without."""
-    names = ("agpt_blk10fwd_kernel", "agpt_blk12bwd_q_kernel", "agpt_blk13bwd_kv_kernel", "agpt_blk10bwd_kernel",
-             "agpt_blk16bwd_carry_kernel", "21trie_bwd_chunk_kernel")
-    calls: dict = {}
+def _listing(images, names):
+    """Instructions of the kernels whose name holds one of `names`."""
+    found: dict = {}
     for img in images:
         text = subprocess.run([LLVM + "llvm-objdump", "-d", "--no-show-raw-insn", "--no-leading-addr", img],
                               capture_output=True, text=True, check=True).stdout
         cur = None
         for line in text.splitlines():
             if line.endswith(">:"):
-                cur = line.split("<")[-1][:-2]
-                if any(n in cur for n in names):
-                    calls[cur] = 0
-                else:
-                    cur = None
-            elif cur and "s_swappc_b64" in line:
-                calls[cur] += 1
-    assert {n for n in names if any(n in k for k in calls)} == set(names)
-    for name, n in calls.items():
-        assert n <= 1, f"{name}: {n} calls"
+                name = line.split("<")[-1][:-2]
+                cur = found.setdefault(name, []) if any(n in name for n in names) else None
+            elif cur is not None and line.strip():
+                cur.append(line.split("//")[0].strip())
+    assert all(any(n in k for k in found) for n in names)
+    return found
+
+
+def test_block_kernels_neither_call_nor_wait_for_a_claim(images):
+    """The block kernels and the reductions behind them: one call, the thread's
+    number at the kernel's start (the workgroup's number and the grid size are
+    read without), and, in the forward and the one-pass backward, no wait behind
+    the atomic that sends for the next claim."""
+    for name, code in _listing(images, ("agpt_blk10fwd_kernel", "agpt_blk12bwd_q_kernel", "agpt_blk13bwd_kv_kernel",
+                                        "agpt_blk10bwd_kernel", "agpt_blk16bwd_carry_kernel",
+                                        "21trie_bwd_chunk_kernel")).items():
+        assert sum("s_swappc_b64" in x for x in code) <= 1, f"{name}: calls"
+        for x, y in zip(code, code[1:] if "agpt_blk10" in name else []):
+            assert not ("global_atomic_add" in x and "vmcnt(0)" in y), f"{name}: waits for its claim"
